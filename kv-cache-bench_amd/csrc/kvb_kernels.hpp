@@ -167,6 +167,9 @@ struct ReduceParams {
     int len_cap;                // as DecodeParams::len_cap
 };
 
+// Tokens one workgroup of the naive passes owns.
+constexpr int kNaiveChunk = 128;
+
 struct NaiveParams {
     const float* q;
     const void* k;              // [B][Hkv][max_len][D]
@@ -178,6 +181,9 @@ struct NaiveParams {
     int num_kv_heads;
     int max_len;
     float scale;
+    int chunks;                 // max(1, ceil(max_len / kNaiveChunk))
+    float* part;                // [B][H][chunks][D]: a chunk's share of the output
+    float2* stats;              // [B][H][chunks]: a chunk's (max score, exp-sum)
 };
 
 // Timing marks of a launch: `start` is recorded on the stream right before the kernel, `stop` is

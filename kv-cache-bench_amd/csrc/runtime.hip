@@ -785,10 +785,17 @@ int kvb_run_naive(const kvb_naive_args* a, double* ms) {
     if (int st = kvb_check_naive(a)) return st;
     if (int st = ensure_device()) return st;
     if (a->batch == 0) return KVB_OK;
-    const size_t need = (size_t)a->batch * a->num_heads * (size_t)std::max(a->max_len, 1) * sizeof(float);
+    // scores [rows][max_len], then each chunk's parts of the output and (max, sum), 16-byte aligned
+    const size_t rows = (size_t)a->batch * a->num_heads;
+    const size_t chunks = ((size_t)std::max(a->max_len, 1) + kvbk::kNaiveChunk - 1) / kvbk::kNaiveChunk;
+    const size_t score_floats = (rows * (size_t)std::max(a->max_len, 1) + 3) / 4 * 4;
+    const size_t part_floats = rows * chunks * (size_t)a->head_dim;
+    const size_t need = (score_floats + part_floats + 2 * rows * chunks) * sizeof(float);
     if (int st = grow(&g.scores, &g.scores_bytes, need)) return st;
-    kvbk::NaiveParams p{a->q, a->k, a->v, a->seq_lens, static_cast<float*>(g.scores), a->out,
-                        a->num_heads, a->num_kv_heads, a->max_len, 1.0f / std::sqrt((float)a->head_dim)};
+    float* scores = static_cast<float*>(g.scores);
+    kvbk::NaiveParams p{a->q, a->k, a->v, a->seq_lens, scores, a->out, a->num_heads, a->num_kv_heads, a->max_len,
+                        1.0f / std::sqrt((float)a->head_dim), (int)chunks, scores + score_floats,
+                        reinterpret_cast<float2*>(scores + score_floats + part_floats)};
     hipEvent_t e0, e1;
     if (int st = get_event(&e0)) return st;
     if (int st = get_event(&e1)) return st;
@@ -804,7 +811,8 @@ int kvb_run_attention_fp64(const kvb_naive_args* a, double* ms) {
     if (int st = ensure_device()) return st;
     if (a->batch == 0) return KVB_OK;
     kvbk::NaiveParams p{a->q, a->k, a->v, a->seq_lens, nullptr, a->out,
-                        a->num_heads, a->num_kv_heads, a->max_len, 1.0f / std::sqrt((float)a->head_dim)};
+                        a->num_heads, a->num_kv_heads, a->max_len, 1.0f / std::sqrt((float)a->head_dim), 0, nullptr,
+                        nullptr};
     hipEvent_t e0, e1;
     if (int st = get_event(&e0)) return st;
     if (int st = get_event(&e1)) return st;
