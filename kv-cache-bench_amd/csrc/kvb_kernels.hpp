@@ -251,8 +251,10 @@ struct CacheWriteParams {
     int max_len;
     int quantize;               // 1: fp32 -> int8 with per-(block, KV head) scales
     int len_cap;                // live_len's cap: min(max_len, max_blocks * page_size)
+    FastDiv page_div;           // division by page_size
+    int row_shift;              // log2 of a row's 16-byte words (scatter)
 };
-// grid (Hkv, batch, max_blocks_used): max_blocks_used = ceil(max_len / page)
+// grid (Hkv, batch, runs of tokens or groups of logical blocks): max_blocks_used = ceil(max_len / page)
 hipError_t launch_write_paged(const CacheWriteParams& p, int batch, int max_blocks_used, hipStream_t s,
                               const Marks& m = {});
 

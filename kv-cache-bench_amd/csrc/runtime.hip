@@ -755,6 +755,8 @@ int kvb_write_paged(const kvb_cache_args* a, double* ms) {
     p.max_blocks = a->max_blocks;
     p.max_len = a->max_len;
     p.quantize = a->kv_type == KVB_KV_I8;
+    p.page_div = kvbk::make_fast_div((uint32_t)a->page_size);
+    while ((16 << p.row_shift) < p.head_dim * p.elem_size) ++p.row_shift;
     p.len_cap = (int)std::min((long long)a->max_len, (long long)a->max_blocks * a->page_size);
     hipEvent_t e0, e1;
     if (int st = get_event(&e0)) return st;

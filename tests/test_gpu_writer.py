@@ -68,6 +68,23 @@ def test_writer_matches_host_bytes(gpu, kv, page):
     check_writer(kvb, w, page, page * 5 + 1, 2.0)
 
 
+# One page around each limit of the quantiser's forms (a wave per block up to 2048 values, a workgroup
+# with 8 and 16 registers up to 8192 and 16384, two passes past that) and pages that straddle the copy's
+# 16 KB runs, with lengths around the runs' and the blocks' ends.
+@pytest.mark.parametrize("kv,dim,page", [("i8", 64, 32), ("i8", 64, 33), ("i8", 128, 16), ("i8", 128, 17), ("i8", 128, 64),
+                                         ("i8", 128, 65), ("i8", 128, 128), ("i8", 128, 129), ("f16", 128, 7),
+                                         ("f16", 64, 100), ("f32", 128, 31), ("f32", 64, 200)])
+def test_writer_form_limits(gpu, kv, dim, page):
+    kvb = gpu
+    lens = [page, 0, page + 1, 4 * page - 1, 31, 32, 33, 63, 65, 127, 128, 129, 257]
+    w = kvb.Workload(kvb.Shape(len(lens), 4, 2, dim), kv, lens, seed=page, varied=(kv == "i8"))
+    if kv == "i8":  # ties of the quantiser (scale 1/8), a zero block, and rows whose division is inexact
+        w.k[0, 0] = ((np.arange(w.k[0, 0].size) % 253 - 126) / 16.0).reshape(w.k[0, 0].shape)
+        w.k[0, 0, 0, 0] = 127 / 8.0
+        w.k[0, 1] = 0.0
+    check_writer(kvb, w, page, page + 3, 1.5)
+
+
 @pytest.mark.parametrize("kv", ["f16", "i8"])
 def test_writer_c5_shape(gpu, kv):
     """BASELINE c5's ragged batch (page 64, 3x pool, N(0,1)): the GPU-written pool and scales are the
