@@ -84,7 +84,10 @@ typedef struct kvb_paged_args {
     int page_size;    /* tokens per physical block */
     int max_blocks;   /* row stride of block_table */
     int max_len;      /* longest sequence; sizes the split-K workspace; 0: every output is 0 */
-    int part_tokens;  /* split-K partition size in tokens, 0 = kvb_auto_part_tokens() */
+    int part_tokens;  /* split-K partition size in tokens; 0: kvb_auto_part_tokens() with a workspace of
+                         the caller's, else the library's choice: each sequence cut evenly into partitions of
+                         at least kvb_auto_part_tokens() tokens (or all of it), sized for the batch's lengths.
+                         The sums then run in another order than with an explicit size */
     int share_kv;     /* 1: one workgroup serves every query head of a KV head (reads K/V once per
                          group); 0: one workgroup per query head (the GQA ablation) */
     const float* q;              /* device, float [B][H][D] */
@@ -110,7 +113,8 @@ typedef struct kvb_paged_args {
     size_t workspace_bytes;
 } kvb_paged_args;
 
-/* Split-K partition size used when part_tokens == 0 (auto_part_tokens, src/metal_attn.hpp:43-51):
+/* The reference's rule for part_tokens == 0 (auto_part_tokens, src/metal_attn.hpp:43-51), which sizes
+ * the workspace there (kvb_paged_max_parts, kvb_paged_workspace_bytes):
  * the largest power of two in [64, 512] with batch * Hkv * ceil(max_len / part) >= 512. */
 int kvb_auto_part_tokens(int batch, int num_kv_heads, int max_len);
 /* Partitions per (sequence, head) in the workspace: max(1, ceil(max_len / part)) with part

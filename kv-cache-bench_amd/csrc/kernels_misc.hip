@@ -18,7 +18,8 @@ constexpr float kNegBigR = -1e30f;
 template <int D>
 __global__ __launch_bounds__(D) void paged_reduce_kernel(ReduceParams p) {
     const int h = blockIdx.x, b = blockIdx.y, d = threadIdx.x, H = p.num_heads;
-    const int parts = (live_len(p.seq_lens, b, p.len_cap) + p.part_tokens - 1) / p.part_tokens;  // <= max_parts
+    const int len = live_len(p.seq_lens, b, p.len_cap), part = seq_part(p.split, len);
+    const int parts = len > 0 ? (len + part - 1) / part : 0;  // <= max_parts
     float* o = p.out + ((size_t)b * H + h) * D;
     if (parts <= 0) {
         o[d] = 0.0f;

@@ -78,6 +78,25 @@ __device__ __forceinline__ int fast_div(int n, FastDiv f) {
     return f.mul ? (int)(__umulhi((uint32_t)n, f.mul) >> f.shift) : n;
 }
 
+// The split of a sequence into partitions. Plain: partitions of part_tokens tokens, the last one
+// partial. Even: as many partitions as part_tokens tokens each would need, all of one size but the
+// last (a multiple of kEvenTokens, so that every wave of a workgroup gets as many tiles), so that no
+// short remainder is left: the library's choice where the caller leaves the partition to it (runtime.hip).
+constexpr int kEvenTokens = 128;
+struct SplitParams {
+    int part_tokens;
+    int even;
+    FastDiv part_div;           // division by part_tokens
+};
+// Tokens per partition of a sequence of len tokens, 1 <= len; ceil(len / that) <= ceil(len / part_tokens).
+__host__ __device__ __forceinline__ int even_part(int len, int n) {
+    return n <= 1 ? (len + kEvenTokens - 1) / kEvenTokens * kEvenTokens
+                  : ((len + n - 1) / n + kEvenTokens - 1) / kEvenTokens * kEvenTokens;
+}
+__device__ __forceinline__ int seq_part(const SplitParams& s, int len) {
+    return s.even ? even_part(len, fast_div(len + s.part_tokens - 1, s.part_div)) : s.part_tokens;
+}
+
 struct DecodeParams {
     const float* q;             // [B][H][D]
     const void* k;              // [blocks][Hkv][page][D]
@@ -123,14 +142,20 @@ struct DecodeParams {
     // kernels only (the others serve QG heads). Last, so that it leaves the other fields' offsets
     // in the kernel arguments as they were.
     int qg;
-    // Nonzero (any-page path only, page_size or part_tokens not a multiple of kTile): a workgroup's
-    // range touches at most kTableStage blocks, so the STAGE kernel copies their ids into LDS.
+    // Any-page path only (page_size or part_tokens not a multiple of kTile): the most blocks a
+    // workgroup's range touches, where the STAGE kernel copies them into LDS (at most kTableStage); else 0.
     int table_in_lds;
+    int quads;                  // page_size and the partition are multiples of 4: 4 aligned tokens share a page
+    SplitParams split;          // split.part_tokens == part_tokens
 };
 
 // Block ids the any-page kernel stages in LDS per workgroup (16 KB): a 4096-token partition at any
 // page size, page 1 included.
 constexpr int kTableStage = 4096;
+// Ranges of up to this many blocks run a build that stages no more, where LDS limits the workgroups
+// per CU otherwise: int8, which stages each block's scales too (12 bytes a block: 6 KB against 48), and
+// fp32, whose V tiles take 64 KB (two workgroups per CU against one).
+constexpr int kTableStageSmall = 512;
 
 // Blocks of one partition that paged_decode holds in lanes: one per lane of one VGPR (and, for int8,
 // one VGPR each for the K and V scales). With more, it reads the block table per tile instead.
@@ -163,7 +188,7 @@ struct ReduceParams {
     float* out;                 // [B][H][D]
     int num_heads;
     int max_parts;
-    int part_tokens;
+    SplitParams split;
     int len_cap;                // as DecodeParams::len_cap
 };
 

@@ -207,7 +207,9 @@ struct KvT<KV_F32, D> {
     static constexpr int LDS_ESZ = 4;
     __device__ static int kdoff(int c, int q4) { return 16 * c + 4 * q4; }
     __device__ static int dslot(int j, int q4, int /*s*/) { return 16 * (j >> 2) + 4 * q4 + (j & 3); }
-    __device__ static int swz(int t) { return 4 * ((t >> 2) & 1); }
+    // a read takes 16 adjacent floats of rows 4 q4 + u, q4 = 0..3: four 64-byte runs at distinct offsets
+    // mod 256 bytes (all the banks)
+    __device__ static int swz(int t) { return 4 * ((t >> 2) & 3); }
 };
 
 // Raw registers of one 32-token tile.
@@ -217,6 +219,7 @@ struct TileRegs {
     uint4 k[2][T::KLOADS];
     uint4 v[2][T::NV];
     // int8: K and V scales of the tokens this lane holds in the score layout (FAST: one per half)
+    // (any page with the block ids in LDS: read from there instead)
     float ks[KIND == KV_I8 ? 8 : 1], vs[KIND == KV_I8 ? 8 : 1];
     // FAST with the partition's blocks in lanes: each half's block, relative to the partition's first
     int rel[2];
@@ -254,8 +257,18 @@ __device__ __forceinline__ int wave_inclusive_sum(int x) {
 // lengths in seq_lens (clamped by live_len) make a different number of items, the two copies
 // disagree: every workgroup then gets no item and the launch does nothing, rather than leave some
 // partitions unlaunched and their group's arrival counter short of its count for later launches.
-__device__ __forceinline__ WorkItem ragged_item(const int32_t* seq_lens, int batch, int part_tokens, int len_cap,
+// Even splits (SplitParams::even) keep the order: full partitions (of each sequence's own size) in
+// sequence order, then the last partial ones, longest first. (All of a sequence's partitions in sequence
+// order left the remainders among the full ones: 40 ragged fp32 sequences up to 4096 tokens, page 64,
+// 512-token partitions, ran 124 us that way and 113 this way.)
+__device__ __forceinline__ WorkItem ragged_item(const int32_t* seq_lens, int batch, const SplitParams& sp, int len_cap,
                                                 int i, int items) {
+    const int part_tokens = sp.part_tokens;
+    // a sequence's full partitions
+    auto full = [&](int len) {
+        if (!sp.even) return fast_div(len, sp.part_div);
+        return len > 0 ? len / seq_part(sp, len) : 0;
+    };
     constexpr int E = kRaggedMaxBatch / 64;
     const int lane = threadIdx.x & 63;
     const int ne = (batch + 63) >> 6;
@@ -265,7 +278,7 @@ __device__ __forceinline__ WorkItem ragged_item(const int32_t* seq_lens, int bat
     // full partitions, in sequence order: an exclusive scan of len / part_tokens
     int before = 0;
     for (int e = 0; e < E && e < ne; ++e) {
-        const int f = len[e] / part_tokens;
+        const int f = full(len[e]);
         const int s = wave_inclusive_sum(f);
         const int excl = before + s - f;
         const unsigned long long hit = __ballot(f > 0 && excl <= i && i < excl + f);
@@ -280,7 +293,7 @@ __device__ __forceinline__ WorkItem ragged_item(const int32_t* seq_lens, int bat
     int npart = 0, nempty = 0;
     unsigned key[E];
     for (int e = 0; e < E; ++e) {
-        const int rem = len[e] % part_tokens;
+        const int rem = len[e] > 0 ? len[e] - full(len[e]) * seq_part(sp, len[e]) : 0;
         key[e] = (e < ne && rem > 0) ? ((unsigned)rem << 16) | (0xFFFFu - (unsigned)(64 * e + lane)) : 0u;
         if (e < ne) {
             npart += __popcll(__ballot(key[e] != 0u));
@@ -306,7 +319,7 @@ __device__ __forceinline__ WorkItem ragged_item(const int32_t* seq_lens, int bat
             int lb = 0;
             for (int e = 0; e < E && e < ne; ++e)
                 if (e == (b >> 6)) lb = __builtin_amdgcn_readlane(len[e], b & 63);
-            r = WorkItem{b, lb / part_tokens};
+            r = WorkItem{b, full(lb)};
         } else {
             // empty sequences, in sequence order
             int k = j - npart;
@@ -342,7 +355,7 @@ __device__ __forceinline__ WorkItem ragged_item(const int32_t* seq_lens, int bat
 // each tile is read by HS waves, the first from HBM and the others mostly from the CU's caches, with
 // ordinary loads; fp16: the stream's two waves load half a tile each and share it through LDS (SHL).
 template <int KIND, int D, int QG, bool FAST, bool LOADS = false, bool PAIR = false, bool PART = false,
-          bool SHARE = false, bool STAGE = false>
+          bool SHARE = false, int STAGE = 0>
 __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdgpu_waves_per_eu(
     decode_wg_waves(KIND, QG) > 4 ? 2
     : decode_shape(KIND, QG).qw > 8 ? 1
@@ -445,7 +458,7 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
     }
     int part = bz * G, b = by;  // part: the workgroup's first partition
     if (p.ragged_items) {
-        const WorkItem it = ragged_item(p.seq_lens, p.batch, p.part_tokens, p.len_cap, by, gridDim.y);
+        const WorkItem it = ragged_item(p.seq_lens, p.batch, p.split, p.len_cap, by, gridDim.y);
         if (it.b < 0 || it.b >= p.batch || it.part >= p.max_parts) return;  // uniform, before any barrier
         b = it.b;
         part = it.part;
@@ -455,7 +468,8 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
     const int NQ = PART ? p.qg : QG;
     const int h0 = bx * NQ;
     const int len = live_len(p.seq_lens, b, p.len_cap);  // nparts <= max_parts, t1 <= max_blocks * P
-    const int t0 = part * p.part_tokens;
+    const int PT = seq_part(p.split, len);  // tokens per partition of this sequence
+    const int t0 = part * PT;
     const int H = p.num_heads, Hkv = p.num_kv_heads, P = p.page_size;
     if (t0 >= len) {  // uniform over the workgroup, before any barrier
         // fused merge: an empty sequence attends to nothing, its output is exactly 0
@@ -463,8 +477,8 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
             for (int idx = threadIdx.x; idx < NQ * D; idx += 64 * W) p.out[((size_t)b * H + h0) * D + idx] = 0.0f;
         return;
     }
-    const int t1 = min(len, t0 + G * p.part_tokens);
-    const int ng = PAIR ? (t1 - t0 + p.part_tokens - 1) / p.part_tokens : 1;  // partitions holding tokens
+    const int t1 = min(len, t0 + G * PT);
+    const int ng = PAIR ? (t1 - t0 + PT - 1) / PT : 1;  // partitions holding tokens
     const int kvh = h0 / p.group;
 
     const int lane = threadIdx.x & 63;
@@ -493,15 +507,25 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
     // ids are copied into LDS once instead, and a lookup is an LDS read. (MI355X, c4's size with
     // 8-token pages: see the tile walk.)
     static_assert(!STAGE || !FAST, "STAGE is an any-page variant");
-    __shared__ int s_tab[STAGE ? kTableStage : 1];
+    // int8: their K and V scales as well, read by compute_tile. As loads of each tile, 8 tokens' scales
+    // per lane, they were twice the tile's K and V load instructions and held 32 VGPRs.
+    __shared__ int s_tab[STAGE ? STAGE : 1];
+    __shared__ float2 s_sc[STAGE && KIND == KV_I8 ? STAGE : 1];
     const int tb0 = fast_div(t0, p.page_div);
-    if constexpr (STAGE) {
-        const int nbs = fast_div(t1 - 1, p.page_div) - tb0 + 1;  // <= kTableStage (host-checked)
-        for (int i = threadIdx.x; i < nbs; i += 64 * W) s_tab[i] = p.block_table[(size_t)b * p.max_blocks + tb0 + i];
+    if constexpr (STAGE != 0) {
+        const int nbs = fast_div(t1 - 1, p.page_div) - tb0 + 1;  // <= STAGE (host-checked)
+        for (int i = threadIdx.x; i < nbs; i += 64 * W) {
+            const int id = p.block_table[(size_t)b * p.max_blocks + tb0 + i];
+            s_tab[i] = id;
+            if constexpr (KIND == KV_I8) {
+                const size_t slot = (size_t)max(id, 0) * Hkv + kvh;
+                s_sc[i] = make_float2(p.k_scale[slot], p.v_scale[slot]);
+            }
+        }
         __syncthreads();
     }
     auto block_of = [&](int bi) -> int {
-        if constexpr (STAGE) return s_tab[bi - tb0];
+        if constexpr (STAGE != 0) return s_tab[bi - tb0];
         else return bt[bi];
     };
     const const_f32 ksc = (const_f32)p.k_scale, vsc = (const_f32)p.v_scale;
@@ -530,7 +554,16 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
     // against 186.0-186.7, c4's shape in int8 46.9-47.1 against 47.9, c3 even. fp16 keeps the
     // interleaved order: K first made c2 28.0-28.1 us against 27.6-27.7, and c5 fp16 339 against 335.
     constexpr bool KFIRST = FAST && KIND == KV_I8;
-    auto load_tile = [&](R& r, int tt) {
+    // 16 bytes of a row through its own address (any page size), with the cache policy of kKvPolicy
+    auto row_load = [&](const char* at) -> uint4 {
+        const u32x4_t* src = reinterpret_cast<const u32x4_t*>(at);
+        if constexpr (kKvPolicy == kNonTemporal) return __builtin_bit_cast(uint4, __builtin_nontemporal_load(src));
+        else return __builtin_bit_cast(uint4, *src);
+    };
+    // dok, dov: the K rows, the V rows (fp32 loads the two at different places of its walk)
+    auto load_rows = [&](R& r, int tt, auto dok, auto dov) {
+        constexpr bool DOK = decltype(dok)::value, DOV = decltype(dov)::value;
+        static_assert((DOK && DOV) || !KFIRST, "int8 loads whole tiles");
         int braw = 0, off = 0;  // FAST: the block id of the half tile and its first row in the page
         __amdgpu_buffer_rsrc_t rvh[KFIRST ? 2 : 1];  // KFIRST: each half's V resource, for after both K
         for (int h = 0; h < 2; ++h) {
@@ -562,12 +595,13 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
                     const_cast<char*>(kbase + row0 * D * T::ESZ), (short)0, nbytes, 0x00020000);
                 const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
                     const_cast<char*>(vbase + row0 * D * T::ESZ), (short)0, nbytes, 0x00020000);
-                for (int m = 0; m < T::KLOADS; ++m)
-                    r.k[h][m] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                              rk, (c * D + T::kdoff(m, q4)) * T::ESZ, 0, kKvPolicy));
+                if constexpr (DOK)
+                    for (int m = 0; m < T::KLOADS; ++m)
+                        r.k[h][m] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                                  rk, (c * D + T::kdoff(m, q4)) * T::ESZ, 0, kKvPolicy));
                 if constexpr (KFIRST) {
                     rvh[h] = rv;
-                } else {
+                } else if constexpr (DOV) {
                     for (int i = 0; i < NV; ++i)
                         r.v[h][i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
                                                                   rv, (i * (64 / VL) + lane / VL) * D * T::ESZ + (lane % VL) * 16, 0, kKvPolicy));
@@ -593,10 +627,12 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
                 const bool kval = tk < t1 && kid >= 0;
                 const size_t krow = ((size_t)max(kid, 0) * Hkv + kvh) * P + (tks - kbi * P);
                 const char* kb = kbase + krow * D * T::ESZ;
-                for (int m = 0; m < T::KLOADS; ++m) {
-                    const uint4 x = *reinterpret_cast<const uint4*>(kb + T::kdoff(m, q4) * T::ESZ);
-                    r.k[h][m] = kval ? x : make_uint4(0, 0, 0, 0);
-                }
+                if constexpr (DOK)
+                    for (int m = 0; m < T::KLOADS; ++m) {
+                        const uint4 x = row_load(kb + T::kdoff(m, q4) * T::ESZ);
+                        r.k[h][m] = kval ? x : make_uint4(0, 0, 0, 0);
+                    }
+                if constexpr (!DOV) continue;
                 for (int i = 0; i < NV; ++i) {
                     const int tv = th + i * (64 / VL) + lane / VL;
                     const int tvs = tv < t1 ? tv : t0;
@@ -604,10 +640,10 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
                     const int vid = block_of(vbi);
                     const bool vval = tv < t1 && vid >= 0;
                     const size_t vrow = ((size_t)max(vid, 0) * Hkv + kvh) * P + (tvs - vbi * P);
-                    const uint4 x = *reinterpret_cast<const uint4*>(vbase + vrow * D * T::ESZ + (lane % VL) * 16);
+                    const uint4 x = row_load(vbase + vrow * D * T::ESZ + (lane % VL) * 16);
                     r.v[h][i] = vval ? x : make_uint4(0, 0, 0, 0);
                 }
-                if constexpr (KIND == KV_I8) {
+                if constexpr (KIND == KV_I8 && !STAGE) {
                     for (int i = 0; i < 4; ++i) {  // the score-layout tokens th + 4*q4 + i of this lane
                         const int ts = th + 4 * q4 + i;
                         const int tss = ts < t1 ? ts : t0;
@@ -624,6 +660,7 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
                     r.v[h][i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
                                                               rvh[h], (i * (64 / VL) + lane / VL) * D * T::ESZ + (lane % VL) * 16, 0, kKvPolicy));
     };
+    auto load_tile = [&](R& r, int tt) { load_rows(r, tt, std::true_type{}, std::true_type{}); };
 
     // ---- SHL: this wave's half of a tile, K rows (split 0) or V rows (split 1), into x[h][m]: the
     // rows and buffer ranges of load_tile, each lane's row and byte of the one or the other (for
@@ -661,7 +698,7 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
                     const int bi = fast_div(tks, p.page_div);
                     const int id = block_of(bi);
                     const size_t row = ((size_t)max(id, 0) * Hkv + kvh) * P + (tks - bi * P);
-                    const uint4 v = *reinterpret_cast<const uint4*>(hbase + row * D * T::ESZ + hcol(m));
+                    const uint4 v = row_load(hbase + row * D * T::ESZ + hcol(m));
                     x[h][m] = tk < t1 && id >= 0 ? v : make_uint4(0, 0, 0, 0);
                 }
             }
@@ -724,7 +761,7 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
             __builtin_amdgcn_sched_barrier(0);
         }
     } else {
-        for (int k = 0; k + 1 < NBUF; ++k) {
+        for (int k = 0; k + 1 < NBUF || k == 0; ++k) {
             load_tile(r[k], t0 + (it + k * TS) * kTok);
             // (in buffer order, as the loop issues them: the loop head is entered from here and from the
             // back edge, and the wait for buffer 0 there can leave the later buffers in flight only if
@@ -830,6 +867,7 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
     // and at the end they are scaled by 2^ve. (ve starts below every float exponent: 2^-160 is 0.)
     float vdown = 1.0f;
     int ve = -160;
+    float vlimit = 0.0f;  // 2^ve
 
     // ---- V tile -> LDS as stored (row-major, swizzled 16-byte chunks; int8 is widened to fp16 only
     // after the transposing read)
@@ -856,7 +894,8 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
         for (int mb = 0; mb < NMB; ++mb) acc[a][mb] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
     uint32_t lsink = 0;  // LOADS: what the tiles' registers XOR to
-    auto compute_tile = [&](const R& r, int tt) {
+    // v_done, k_done: called once the tile's V rows, its K rows, are out of the registers
+    auto compute_tile = [&](const R& r, int tt, auto v_done, auto k_done) {
         if constexpr (LOADS) {
             for (int h = 0; h < 2; ++h) {
                 for (int mm = 0; mm < T::KLOADS; ++mm) lsink ^= r.k[h][mm].x ^ r.k[h][mm].y ^ r.k[h][mm].z ^ r.k[h][mm].w;
@@ -866,9 +905,26 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
                 for (int j = 0; j < 2; ++j)
                     lsink ^= __builtin_bit_cast(uint32_t, r.ks[j]) ^ __builtin_bit_cast(uint32_t, r.vs[j]);
             (void)tt;
+            v_done();
+            k_done();
             return;
         }
+        // int8, staged: the scales of the lane's tokens (tokens past t1: the range's first, live, token)
+        float2 sc[KIND == KV_I8 && STAGE ? 8 : 1];
+        if constexpr (KIND == KV_I8 && STAGE) {
+            auto scale_of = [&](int t) { return s_sc[fast_div(t < t1 ? t : t0, p.page_div) - tb0]; };
+            for (int h = 0; h < 2; ++h) {
+                const int ts = tt + h * kHalf + 4 * q4;
+                if (p.quads) {  // the lane's 4 tokens lie in one page (the last live one may end it early)
+                    const float2 x = scale_of(ts);
+                    for (int i = 0; i < 4; ++i) sc[4 * h + i] = x;
+                } else {
+                    for (int i = 0; i < 4; ++i) sc[4 * h + i] = scale_of(ts + i);
+                }
+            }
+        }
         if constexpr (!SHL) store_v(r);  // (SHL: the tile is in LDS already)
+        v_done();
         // S^T = K Q^T for both halves. S[a][h]: a = 0 the column's part (COLH: the high part,
         // int8 d0 + d2 / 2^14), a = 1 (COLH) the low part (int8 d1 / 2^7): the values columns 2h and
         // 2h + 1 hold in the two-column layout.
@@ -905,6 +961,7 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
                 }
             }
         }
+        k_done();
         // int8, FAST: the scales of the two halves (the first's for both with tile_in_page), from the
         // lanes that hold them when the partition's scales are in lanes
         float ksh[2], vsh[2];
@@ -919,11 +976,22 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
             ksh[1] = (FAST && p.tile_in_page) ? r.ks[0] : r.ks[KIND == KV_I8 ? 1 : 0];
             vsh[1] = (FAST && p.tile_in_page) ? r.vs[0] : r.vs[KIND == KV_I8 ? 1 : 0];
         }
+        // int8, any page: the scales of the lane's token j
+        auto kscale = [&](int j) -> float {
+            if constexpr (KIND == KV_I8 && STAGE) return sc[j].x;
+            else return r.ks[KIND == KV_I8 ? j : 0];
+        };
+        auto vscale = [&](int j) -> float {
+            if constexpr (KIND == KV_I8 && STAGE) return sc[j].y;
+            else return r.vs[KIND == KV_I8 ? j : 0];
+        };
         if constexpr (KIND == KV_I8) {
             float vmx = FAST ? fmaxf(vsh[0], vsh[1]) : 0.0f;
             if constexpr (!FAST) {
-                for (int j = 0; j < 8; ++j) vmx = fmaxf(vmx, r.vs[j]);
-                vmx = wave_max(vmx);
+                for (int j = 0; j < 8; ++j) vmx = fmaxf(vmx, vscale(j));
+                // (no lane's scale at or past 2^ve, on all tiles but a few: no max over the wave either)
+                if (__builtin_amdgcn_ballot_w64(vmx >= vlimit) != 0) vmx = wave_max(vmx);
+                else vmx = 0.0f;
             }
             int e = ve;
             if (vmx > 0.0f) frexpf(vmx, &e);  // vmx < 2^e
@@ -933,6 +1001,7 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
                     for (int mb = 0; mb < NMB; ++mb) acc[a][mb] *= down;
                 ve = e;
                 vdown = ldexpf(1.0f, -e);
+                vlimit = ldexpf(1.0f, e);
             }
         }
         // scores of this lane's 8 tokens for head hh: high + low columns (COLH: parts), scaled,
@@ -945,7 +1014,7 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
                 for (int i = 0; i < 4; ++i) {
                     const int j = 4 * h + i;
                     float f = up;
-                    if constexpr (KIND == KV_I8) f *= FAST ? ksh[h] : r.ks[j];
+                    if constexpr (KIND == KV_I8) f *= FAST ? ksh[h] : kscale(j);
                     if constexpr (COLH) s[j] = (S[0][h][i] + S[NA - 1][h][i]) * f;
                     else s[j] = (S[0][h][i] + dpp<kQuadSwap1>(S[0][h][i])) * f;
                 }
@@ -972,7 +1041,7 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
                 const float pr = __builtin_amdgcn_exp2f(s[j] - mn);
                 psum += pr;
                 float pv = pr;
-                const float xs = KIND == KV_I8 ? (FAST ? vsh[j >> 2] : r.vs[j]) * vdown : 1.0f;
+                const float xs = KIND == KV_I8 ? (FAST ? vsh[j >> 2] : vscale(j)) * vdown : 1.0f;
                 if constexpr (KIND == KV_I8) pv *= xs;
                 if constexpr (F32) {
                     pb32[j] = hl ? 0.0f : pv;
@@ -1086,7 +1155,7 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
     // PAIR: `cur` is the partition of the range (0 or 1) the wave's state belongs to. At its first
     // tile of the second partition the wave moves its state to s_part and starts afresh.
     int cur = 0;
-    const int tpp = p.part_tokens / kTok;  // tiles per partition
+    const int tpp = PT / kTok;  // tiles per partition
     if constexpr (SHL) {
         // Step j: the wave's half of tile j (two steps old) goes to slot j % 2, the half of tile j + 2
         // is issued into its registers, and once both waves of the stream have written their halves
@@ -1130,7 +1199,7 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
                         for (int m = 0; m < NL; ++m)
                             rr.k[h][m] = *reinterpret_cast<const uint4*>(slot + ((h * NL + m) * 64 + lane) * 16);
                     vt = slot + SKB;
-                    compute_tile(rr, t0 + it * kTok);
+                    compute_tile(rr, t0 + it * kTok, [] {}, [] {});
                 }
                 it += TS;
             }
@@ -1144,8 +1213,10 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
 #pragma unroll
         for (int k = 0; k < NBUF; ++k) {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // tile `it` (buffer k) has arrived
-            load_tile(r[(k + NBUF - 1) % NBUF], t0 + (it + (NBUF - 1) * TS) * kTok);
-            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (NBUF > 1) {
+                load_tile(r[(k + NBUF - 1) % NBUF], t0 + (it + (NBUF - 1) * TS) * kTok);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             if constexpr (PAIR && !LOADS) {
                 if (cur == 0 && it >= tpp && it < ntiles) {  // wave-uniform
                     state_to_lds(s_part[wave], s_ml2[wave], s_mt2[LAZY ? wave : 0], true);
@@ -1156,10 +1227,33 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
                         for (int mb = 0; mb < NMB; ++mb) acc[a][mb] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
                     ve = -160;
                     vdown = 1.0f;
+                    vlimit = 0.0f;
                     cur = 1;
                 }
             }
-            compute_tile(r[k], t0 + it * kTok);
+            if constexpr (NBUF > 1) {
+                // A round's later step may lie past the wave's last tile: nothing to compute (fp16, 2 x 512
+                // tokens, one tile per wave: 7.7 us with that step's arithmetic, 6.8 without). int8 at
+                // head_dim 128 keeps it: the branch cost its long walks 3-6% (16 x 8192 tokens 43.8 -> 46.7
+                // us), more than the step costs its short ones.
+                if (k == 0 || (KIND == KV_I8 && FAST && D == 128) || it < ntiles) compute_tile(r[k], t0 + it * kTok, [] {}, [] {});
+            } else {
+                // fp32: one buffer, refilled with the next tile as it is used: V's registers once the V
+                // rows are in LDS, K's once the scores are computed. (Any page: without the branch past
+                // the last tile, in which the selects of rows past t1 would wait for their loads: 54
+                // us against 47 at 16 x 4096 tokens, 2 KV heads, page 24, 1024-token partitions.)
+                const int tn = t0 + (it + TS) * kTok;
+                compute_tile(r[0], t0 + it * kTok,
+                             [&] {
+                                 if (!FAST || tn < t1) load_rows(r[0], tn, std::false_type{}, std::true_type{});
+                                 __builtin_amdgcn_sched_barrier(0);
+                             },
+                             [&] {
+                                 __builtin_amdgcn_sched_barrier(0);
+                                 if (!FAST || tn < t1) load_rows(r[0], tn, std::true_type{}, std::false_type{});
+                                 __builtin_amdgcn_sched_barrier(0);
+                             });
+            }
             it += TS;
         }
     }
@@ -1255,7 +1349,7 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
             const u32x2_t ml = {__builtin_bit_cast(uint32_t, Mt * kLn2), __builtin_bit_cast(uint32_t, Ls)};
             __builtin_amdgcn_raw_buffer_store_b64(ml, rml, eh * p.max_parts * 8, 0, kScopeAgent);
         }
-        if (p.out && len <= p.part_tokens)  // one partition: this is the output
+        if (p.out && len <= PT)  // one partition: this is the output
             *reinterpret_cast<float4*>(p.out + ((size_t)b * H + h0 + eh) * D + 4 * ed) = r;
     }
 #ifdef KVB_WG_TIMESTAMPS
@@ -1272,7 +1366,7 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
         st[7] = wg_where();
     }
 #endif
-    if (!p.out || len <= p.part_tokens) return;
+    if (!p.out || len <= PT) return;
 
     // ---- fused merge (src/kernels.metal:123-147): the last workgroup of this (sequence, head
     // group) to arrive (the counter counts partitions: each workgroup adds the ng it wrote) weighs
@@ -1284,7 +1378,7 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
     // count came back. An agent-scope release/acquire pair would instead write back and invalidate
     // the whole L2 of the XCD in every workgroup (buffer_wbl2 / buffer_inv): 140 us per c4 step.
     __shared__ int s_last;
-    const int nparts = (len + p.part_tokens - 1) / p.part_tokens;
+    const int nparts = (len + PT - 1) / PT;
     int* counter = p.counters + (size_t)b * gridDim.x + bx;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -1443,14 +1537,14 @@ hipError_t loads_only_lds(size_t* lds) {
     return hipSuccess;
 }
 
-template <int KIND, int D, int QG, bool FAST, bool PAIR, bool PART, bool SHARE, bool STAGE = false>
+template <int KIND, int D, int QG, bool FAST, bool PAIR, bool PART, bool SHARE, int STAGE = 0>
 hipError_t launch_one(const DecodeParams& p, int batch, hipStream_t s, const Marks& m) {
     if (m.describe) {  // the demangled name of the instantiation below, as rocprofv3 prints it
         auto tf = [](bool x) { return x ? "true" : "false"; };
         const bool loads = FAST && p.loads_only;
         std::snprintf(m.describe, m.describe_cap,
-                      "void kvbk::paged_decode_kernel<%d, %d, %d, %s, %s, %s, %s, %s, %s>(kvbk::DecodeParams)", KIND, D,
-                      QG, tf(FAST), tf(loads), tf(PAIR), tf(PART), tf(SHARE), tf(!loads && STAGE));
+                      "void kvbk::paged_decode_kernel<%d, %d, %d, %s, %s, %s, %s, %s, %d>(kvbk::DecodeParams)", KIND, D,
+                      QG, tf(FAST), tf(loads), tf(PAIR), tf(PART), tf(SHARE), loads ? 0 : STAGE);
         return hipSuccess;
     }
     const int gz = PAIR ? (p.max_parts + 1) / 2 : p.max_parts;
@@ -1475,7 +1569,10 @@ template <int KIND, int D, int QG, bool PART, bool SHARE = false>
 hipError_t launch_qg(bool fast, const DecodeParams& p, int batch, hipStream_t s, const Marks& m) {
     if (!fast) {
         if (p.pair) return hipErrorInvalidValue;
-        return p.table_in_lds ? launch_one<KIND, D, QG, false, false, PART, SHARE, true>(p, batch, s, m)
+        if constexpr (KIND != KV_F16)
+            if (p.table_in_lds && p.table_in_lds <= kTableStageSmall)
+                return launch_one<KIND, D, QG, false, false, PART, SHARE, kTableStageSmall>(p, batch, s, m);
+        return p.table_in_lds ? launch_one<KIND, D, QG, false, false, PART, SHARE, kTableStage>(p, batch, s, m)
                               : launch_one<KIND, D, QG, false, false, PART, SHARE>(p, batch, s, m);
     }
     if constexpr (KIND != KV_F32 && decode_shape(KIND, QG).hs == 1) {

@@ -8,6 +8,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <iterator>
 #include <string>
 #include <utility>
 #include <vector>
@@ -158,12 +159,20 @@ int max_parts_of(const kvb_paged_args* a) {
     return std::max(1, (int)(((long long)a->max_len + part - 1) / part));
 }
 
+// How a step cuts its sequences into partitions.
+struct Split {
+    int part;       // tokens per partition, or (even) at most that many
+    int max_parts;  // partitions of max_len tokens: the workspace's stride, the plain grid's z
+    bool even;      // SplitParams::even
+};
+Split split_of(const kvb_paged_args* a);
+
 // The kernels' cap on a device-side length (live_len): what the block table and the workspace of
 // this launch hold, min(max_blocks * page_size, max_parts * part_tokens). The host copy of the
 // lengths has been checked against both; the cap keeps the kernels inside the buffers if the device
 // copy disagrees.
-int len_cap_of(const kvb_paged_args* a) {
-    const long long cap = std::min((long long)a->max_blocks * a->page_size, (long long)max_parts_of(a) * resolve_part(a));
+int len_cap_of(const kvb_paged_args* a, const Split& sp) {
+    const long long cap = std::min((long long)a->max_blocks * a->page_size, (long long)sp.max_parts * sp.part);
     return (int)std::min<long long>(cap, 0x7fffffff);
 }
 
@@ -235,26 +244,34 @@ struct StepMarks {
     kvbk::Marks step, decode, reduce;
 };
 
+// Partitions of a sequence of len tokens.
+long long parts_of(int len, const Split& sp) {
+    if (len <= 0) return 0;
+    long long part = sp.part;
+    if (sp.even) part = kvbk::even_part(len, (int)(((long long)len + sp.part - 1) / sp.part));
+    return (len + part - 1) / part;
+}
+
 // Work items of a ragged batch in the kernel's longest-first order (one per partition holding
 // tokens, one per empty sequence), or 0 for the plain (sequence, partition) grid: sequences of equal
 // length gain nothing from reordering, and the order needs one lane per sequence.
-int ragged_items(const kvb_paged_args* a, int part) {
-    if (a->batch < 2 || a->batch > kvbk::kRaggedMaxBatch || part >= 65536) return 0;
+int ragged_items(const kvb_paged_args* a, const Split& sp) {
+    if (a->batch < 2 || a->batch > kvbk::kRaggedMaxBatch || sp.part >= 65536) return 0;
     const int32_t* lens = a->host_seq_lens;
     bool equal = true;
     long long items = 0;
     for (int b = 0; b < a->batch; ++b) {
         equal = equal && lens[b] == lens[0];
-        items += std::max(1LL, ((long long)lens[b] + part - 1) / part);
+        items += std::max(1LL, parts_of(lens[b], sp));
     }
     return equal || items > 65535 ? 0 : (int)items;
 }
 
 // counters: the fused merge's arrival counters (zero, at least B * H / qg ints), or null for the
 // library's own (grown on demand).
-int enqueue_paged(const kvb_paged_args* a, float* part_out, float2* part_ml, bool fused, const StepMarks& mk,
-                  bool loads_only = false, int* counters = nullptr) {
-    const int part = resolve_part(a);
+int enqueue_paged(const kvb_paged_args* a, const Split& sp, float* part_out, float2* part_ml, bool fused,
+                  const StepMarks& mk, bool loads_only = false, int* counters = nullptr) {
+    const int part = sp.part;
     const int qg = query_heads_per_group(a);
     kvbk::DecodeParams p{};
     p.q = a->q;
@@ -274,12 +291,13 @@ int enqueue_paged(const kvb_paged_args* a, float* part_out, float2* part_ml, boo
     p.page_div = kvbk::make_fast_div((uint32_t)a->page_size);
     p.tile_in_page = a->page_size % 32 == 0 && part % 32 == 0;
     p.max_blocks = a->max_blocks;
-    p.max_parts = max_parts_of(a);
+    p.max_parts = sp.max_parts;
     p.part_tokens = part;
-    p.len_cap = len_cap_of(a);
+    p.split = {part, sp.even ? 1 : 0, kvbk::make_fast_div((uint32_t)part)};
+    p.len_cap = len_cap_of(a, sp);
     p.qscale = (1.0f / std::sqrt((float)a->head_dim)) * 1.4426950408889634f;
     p.batch = a->batch;
-    p.ragged_items = ragged_items(a, part);
+    p.ragged_items = ragged_items(a, sp);
     p.loads_only = loads_only;
     // fused merge when the group's partition (m, l) pairs fit its LDS staging; a workgroup with more
     // output chunks than threads merges in the one-round-trip form only (at most 16 partitions)
@@ -298,7 +316,8 @@ int enqueue_paged(const kvb_paged_args* a, float* part_out, float2* part_ml, boo
     // which then streams alone); one workgroup per CU was faster (c2 on MI355X, 512 workgroups of 512
     // tokens: 28.3 us per step, against 26.5 us for 256 workgroups of 1024 tokens).
     const long long wgs = (long long)a->batch * (a->num_heads / qg) * p.max_parts;
-    p.pair = fast && a->kv_type != KVB_KV_F32 && !p.ragged_items && p.max_parts >= 2 &&
+    // (an even split has no more workgroups than it means to run at once)
+    p.pair = fast && !sp.even && a->kv_type != KVB_KV_F32 && !p.ragged_items && p.max_parts >= 2 &&
              kvbk::decode_shape(a->kv_type, qg).hs == 1 &&
              part % (2 * kvbk::kTile * kvbk::decode_waves(a->kv_type)) == 0 &&
              (g.pair_mode == KVB_PAIR_ALWAYS || (g.pair_mode == KVB_PAIR_AUTO && wgs >= 2LL * g.cus));
@@ -307,7 +326,8 @@ int enqueue_paged(const kvb_paged_args* a, float* part_out, float2* part_ml, boo
     const long long span = (p.pair ? 2LL : 1LL) * part;
     const long long nb_max = span % a->page_size == 0 ? span / a->page_size : span / a->page_size + 2;
     p.table_in_lanes = fast && nb_max <= kvbk::kLaneBlocks;
-    p.table_in_lds = !fast && nb_max <= kvbk::kTableStage;
+    p.table_in_lds = !fast && nb_max <= kvbk::kTableStage ? (int)nb_max : 0;
+    p.quads = a->page_size % 4 == 0 && part % 4 == 0;
     const kvbk::Marks dm{mk.step.start ? mk.step.start : mk.decode.start, fused ? mk.step.stop : mk.decode.stop,
                          mk.step.describe, mk.step.describe_cap};
     const kvbk::Marks rm{mk.reduce.start, mk.step.stop ? mk.step.stop : mk.reduce.stop};
@@ -326,14 +346,106 @@ int enqueue_paged(const kvb_paged_args* a, float* part_out, float2* part_ml, boo
         return KVB_OK;
     }
     if (fused || loads_only) return KVB_OK;
-    kvbk::ReduceParams r{part_out, part_ml, a->seq_lens, a->out, a->num_heads, p.max_parts, part, p.len_cap};
+    kvbk::ReduceParams r{part_out, part_ml, a->seq_lens, a->out, a->num_heads, p.max_parts, p.split, p.len_cap};
     e = kvbk::launch_paged_reduce(a->head_dim, r, a->batch, g.stream, rm);
     if (e != hipSuccess) return fail(KVB_ERUNTIME, std::string("paged_reduce launch: ") + hipGetErrorString(e));
     return KVB_OK;
 }
 
-int workspace_for(const kvb_paged_args* a, float** part_out, float2** part_ml) {
-    const size_t slots = (size_t)a->batch * a->num_heads * (size_t)max_parts_of(a);
+// The split-K workspace of a step: part_out, then part_ml (kvb_hip.h).
+void layout_workspace(const kvb_paged_args* a, const Split& sp, char* base, float** part_out, float2** part_ml) {
+    const size_t slots = (size_t)a->batch * a->num_heads * (size_t)sp.max_parts;
+    *part_out = reinterpret_cast<float*>(base);
+    *part_ml = reinterpret_cast<float2*>(base + slots * (size_t)a->head_dim * sizeof(float));
+}
+
+// Microseconds that a lone workgroup takes for one round of its four waves (128 tokens), which the
+// latency of its loads and its arithmetic set, not the card's bandwidth: from steps of 40 to 100
+// workgroups on MI355X at partitions of 1024 tokens and more.
+float round_us(int kind, int head_dim, bool fast) {
+    const bool d64 = head_dim == 64;
+    const float t = kind == KVB_KV_I8 ? (d64 ? 1.1f : 0.95f) : kind == KVB_KV_F16 ? (d64 ? 1.1f : 1.5f) : (d64 ? 1.9f : 3.4f);
+    return fast ? t : 1.25f * t;  // (any page size: per-lane addresses and scales)
+}
+
+// The partition where the caller leaves it to the library (part_tokens 0) and the library owns the
+// workspace: kvb_auto_part_tokens, or an even split of at most `part` tokens, a multiple of kEvenTokens
+// and larger than that (so that the workspace sized for the former holds it).
+//
+// kvb_auto_part_tokens, the reference's rule, stops at 512 tokens; a workgroup's prologue, its epilogue
+// and its share of the merge then cost as much as its tokens, and short steps are cut into pieces of
+// two waves' work. The rule here takes the candidate with the least estimated time, from what a step is
+// made of (us):
+//   all:   every item's bytes at the card's rate and kItemUs, spread over the CUs
+//   waves: the same in whole items per CU, as many as the fullest CU has
+//   alone: the longest item by itself, or the CUs' resident workgroups in turn, at round_us
+//   merge: none for one partition; past 16 partitions its longer form
+// The constants minimise the loss against the fastest candidate in a sweep of 62 shapes (batch 1-72,
+// 66-32768 tokens, equal and ragged, groups 1-64, all types, pages 8-64; up to 25 candidates each): 1.4%
+// on average, where kvb_auto_part_tokens loses 16%. E.g. (us, auto / this / best) fp16 1 x 4096:
+// 17.4 / 10.0 / 10.0; fp16 2 x 32768: 51.4 / 46.0 / 46.0; int8 72 ragged up to 16384: 252 / 212 / 208; its
+// worst: fp16 64 ragged up to 2048: 56.4 / 59.2 / 52.5; fp32 8 ragged up to 2048: 20.4 / 23.0 / 20.4.
+Split split_of(const kvb_paged_args* a) {
+    constexpr float kItemUs = 1.5f, kAloneUs = 4.0f, kWavesShare = 0.9f, kRate = 27.0e3f;  // kRate: bytes per us and CU
+    // candidates, in kEvenTokens: every one up to 8, then 4 (3 past 4096 tokens) to a factor of 2
+    constexpr int kSteps[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48, 64, 80, 96, 128};
+    Split sp{resolve_part(a), max_parts_of(a), false};
+    if (a->part_tokens != 0 || a->workspace || a->batch <= 0) return sp;
+    const int32_t* lens = a->host_seq_lens;
+    int longest = 0;
+    long long total = 0;
+    bool equal = true;
+    for (int b = 0; b < a->batch; ++b) {
+        longest = std::max(longest, lens[b]);
+        total += lens[b];
+        equal = equal && lens[b] == lens[0];
+    }
+    if (longest == 0 || (!equal && a->batch > kvbk::kRaggedMaxBatch)) return sp;
+    const int groups = a->num_heads / query_heads_per_group(a), seqs = equal ? 1 : a->batch;
+    const float units = (float)groups * (equal ? (float)a->batch : 1.0f), cus = (float)g.cus;
+    const int esz = a->kv_type == KVB_KV_F32 ? 4 : a->kv_type == KVB_KV_F16 ? 2 : 1;
+    const float tokens = (float)total * (float)groups;
+    const float token_us = 2.0f * a->head_dim * esz / kRate;
+    const float alone_us = round_us(a->kv_type, a->head_dim, a->page_size % kvbk::kTile == 0) / kvbk::kEvenTokens;
+    const float resident = a->kv_type == KVB_KV_I8 ? 3.0f : 2.0f;  // workgroups per CU
+    // (partitions of 64 tokens leave two of the four waves idle: only fp32, whose tiles are twice fp16's,
+    // is ever the faster for them)
+    const bool keep = a->kv_type == KVB_KV_F32 || sp.part >= kvbk::kEvenTokens;
+    float best = 0.0f;
+    int part = 0;
+    for (int i = keep ? -1 : 0; i < (int)std::size(kSteps); ++i) {  // -1: kvb_auto_part_tokens
+        const int cand = i < 0 ? sp.part : kSteps[i] * kvbk::kEvenTokens;
+        if (i >= 0 && cand <= sp.part) continue;
+        // (an estimate: the counts in floating point, summed as integers so that the loop vectorises)
+        const float inv = 1.0f / (float)cand;
+        int n_all = 0, most_i = 0;
+        for (int b = 0; b < seqs; ++b) {
+            const int n = std::max((int)((float)lens[b] * inv + 0.999f), 1);
+            const int each = (int)((float)lens[b] / (float)n + 0.999f);
+            n_all += n;
+            most_i = std::max(most_i, each);
+        }
+        const float items = (float)n_all * units;
+        const int grain = std::min(cand, kvbk::kEvenTokens);
+        const float most = std::min((float)((most_i + grain - 1) / grain * grain), (float)longest);
+        const float mean = tokens / items;
+        const float all = (tokens * token_us + items * kItemUs) / cus;
+        const float waves = items > cus ? std::ceil(items / cus) * (mean * token_us + kItemUs) : most * token_us + kItemUs;
+        const float alone = std::max(most * alone_us + kAloneUs, items / (cus * resident) * (mean * alone_us + kAloneUs));
+        const float parts = std::ceil((float)longest * inv);
+        const float merge = parts <= 1.0f ? 0.0f : parts <= 8.0f ? 1.5f : parts <= 16.0f ? 2.0f : 4.5f + 0.03f * (parts - 16.0f);
+        const float est = std::max(all * (1.0f - kWavesShare) + waves * kWavesShare, alone) + merge;
+        if (part == 0 || est < best) {
+            best = est;
+            part = cand;
+        }
+        if (cand >= longest) break;
+    }
+    if (part <= sp.part) return sp;
+    return Split{part, std::max(1, (int)(((long long)a->max_len + part - 1) / part)), true};
+}
+
+int workspace_for(const kvb_paged_args* a, const Split& sp, float** part_out, float2** part_ml) {
     char* base = nullptr;
     if (a->workspace) {
         base = static_cast<char*>(a->workspace);
@@ -341,8 +453,7 @@ int workspace_for(const kvb_paged_args* a, float** part_out, float2** part_ml) {
         if (int st = grow(&g.ws, &g.ws_bytes, workspace_need(a))) return st;
         base = static_cast<char*>(g.ws);
     }
-    *part_out = reinterpret_cast<float*>(base);
-    *part_ml = reinterpret_cast<float2*>(base + slots * (size_t)a->head_dim * sizeof(float));
+    layout_workspace(a, sp, base, part_out, part_ml);
     return KVB_OK;
 }
 
@@ -403,7 +514,7 @@ int kvb_paged_kernel_name(const kvb_paged_args* a, int loads_only, char* buf, si
     StepMarks mk;
     mk.step.describe = buf;
     mk.step.describe_cap = cap;
-    return enqueue_paged(a, nullptr, nullptr, !loads_only, mk, loads_only != 0);
+    return enqueue_paged(a, split_of(a), nullptr, nullptr, !loads_only, mk, loads_only != 0);
 }
 
 int kvb_run_empty_grid(int workgroups, int threads, double* ms) {
@@ -543,14 +654,15 @@ int kvb_run_paged_steps(const kvb_paged_args* a, int steps, double* ms) {
     if (a->batch == 0 || steps == 0) return KVB_OK;
     float* part_out = nullptr;
     float2* part_ml = nullptr;
-    if (int st = workspace_for(a, &part_out, &part_ml)) return st;
+    const Split sp = split_of(a);
+    if (int st = workspace_for(a, sp, &part_out, &part_ml)) return st;
     hipEvent_t e0, e1;
     if (int st = get_event(&e0)) return st;
     if (int st = get_event(&e1)) return st;
     for (int i = 0; i < steps; ++i) {
         StepMarks mk;
         mk.step = {i == 0 ? e0 : nullptr, i == steps - 1 ? e1 : nullptr};
-        if (int st = enqueue_paged(a, part_out, part_ml, true, mk)) return st;
+        if (int st = enqueue_paged(a, sp, part_out, part_ml, true, mk)) return st;
     }
     return finish(e0, e1, ms);
 }
@@ -589,9 +701,10 @@ int kvb_graph_capture_paged(const kvb_paged_args* a, int steps, void** graph) {
         return cleanup(fail(KVB_ERUNTIME, std::string("graph counter fill: ") + hipGetErrorString(e)));
     if (hipStreamSynchronize(g.stream) != hipSuccess)
         return cleanup(fail(KVB_ERUNTIME, "kvb_graph_capture_paged: stream synchronize failed"));
-    const size_t slots = (size_t)a->batch * a->num_heads * (size_t)max_parts_of(a);
-    float* part_out = reinterpret_cast<float*>(base);
-    float2* part_ml = reinterpret_cast<float2*>(base + slots * (size_t)a->head_dim * sizeof(float));
+    const Split sp = split_of(a);
+    float* part_out = nullptr;
+    float2* part_ml = nullptr;
+    layout_workspace(a, sp, base, &part_out, &part_ml);
     if (a->batch == 0) {  // nothing to capture: an empty graph
         hipGraph_t empty = nullptr;
         if (hipGraphCreate(&empty, 0) != hipSuccess ||
@@ -607,7 +720,7 @@ int kvb_graph_capture_paged(const kvb_paged_args* a, int steps, void** graph) {
     if (hipStreamBeginCapture(g.stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
         return cleanup(fail(KVB_ERUNTIME, "kvb_graph_capture_paged: hipStreamBeginCapture failed"));
     int st = KVB_OK;
-    for (int i = 0; i < steps && st == KVB_OK; ++i) st = enqueue_paged(a, part_out, part_ml, true, StepMarks{}, false, counters);
+    for (int i = 0; i < steps && st == KVB_OK; ++i) st = enqueue_paged(a, sp, part_out, part_ml, true, StepMarks{}, false, counters);
     const hipError_t ce = hipStreamEndCapture(g.stream, &captured);
     if (st != KVB_OK || ce != hipSuccess) {
         if (captured) (void)hipGraphDestroy(captured);
@@ -668,10 +781,11 @@ int kvb_run_paged_noalloc(const kvb_paged_args* a) {
     if (a->batch == 0) return KVB_OK;
     char* base = static_cast<char*>(scratch_of(device));
     if (!base) return fail(KVB_ERUNTIME, "kvb_run_paged_noalloc: no scratch on this device: " + g_scratch_err);
-    const size_t slots = (size_t)a->batch * a->num_heads * (size_t)max_parts_of(a);
-    float* part_out = reinterpret_cast<float*>(base + kScratchCounterBytes);
-    float2* part_ml = reinterpret_cast<float2*>(base + kScratchCounterBytes + slots * (size_t)a->head_dim * sizeof(float));
-    return enqueue_paged(a, part_out, part_ml, true, StepMarks{}, false, reinterpret_cast<int*>(base));
+    const Split sp = split_of(a);
+    float* part_out = nullptr;
+    float2* part_ml = nullptr;
+    layout_workspace(a, sp, base + kScratchCounterBytes, &part_out, &part_ml);
+    return enqueue_paged(a, sp, part_out, part_ml, true, StepMarks{}, false, reinterpret_cast<int*>(base));
 }
 
 int kvb_run_paged_split(const kvb_paged_args* a, double* decode_ms, double* reduce_ms) {
@@ -682,14 +796,15 @@ int kvb_run_paged_split(const kvb_paged_args* a, double* decode_ms, double* redu
     if (a->batch == 0) return KVB_OK;
     float* part_out = nullptr;
     float2* part_ml = nullptr;
-    if (int st = workspace_for(a, &part_out, &part_ml)) return st;
+    const Split sp = split_of(a);
+    if (int st = workspace_for(a, sp, &part_out, &part_ml)) return st;
     hipEvent_t e[4];
     for (auto& x : e)
         if (int st = get_event(&x)) return st;
     StepMarks mk;
     mk.decode = {e[0], e[1]};
     mk.reduce = {e[2], e[3]};
-    if (int st = enqueue_paged(a, part_out, part_ml, false, mk)) return st;
+    if (int st = enqueue_paged(a, sp, part_out, part_ml, false, mk)) return st;
     KVB_HIP(hipEventSynchronize(e[3]));
     float d = 0.0f, r = 0.0f;
     KVB_HIP(hipEventElapsedTime(&d, e[0], e[1]));
@@ -710,13 +825,14 @@ int kvb_run_paged_loads(const kvb_paged_args* a, double* ms) {
     if (a->batch == 0) return KVB_OK;
     float* part_out = nullptr;
     float2* part_ml = nullptr;
-    if (int st = workspace_for(a, &part_out, &part_ml)) return st;
+    const Split sp = split_of(a);
+    if (int st = workspace_for(a, sp, &part_out, &part_ml)) return st;
     hipEvent_t e0, e1;
     if (int st = get_event(&e0)) return st;
     if (int st = get_event(&e1)) return st;
     StepMarks mk;
     mk.decode = {e0, e1};
-    if (int st = enqueue_paged(a, part_out, part_ml, false, mk, true)) return st;
+    if (int st = enqueue_paged(a, sp, part_out, part_ml, false, mk, true)) return st;
     return finish(e0, e1, ms);
 }
 
