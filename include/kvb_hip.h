@@ -129,7 +129,9 @@ size_t kvb_paged_workspace_bytes(const kvb_paged_args* a);
  * kernel serves the whole group from one threadgroup (QG = GROUP, src/metal_attn.mm:64-80); here
  * a wave's score MFMA holds up to 8 heads in two columns each, or 16 in one column each (f16, i8),
  * and a workgroup of 32 heads splits them over two sets of waves that walk the same tiles (f16:
- * each tile loaded once and shared through LDS). Returns -1 on bad arguments
+ * each tile loaded once and shared through LDS). A step of at most 16 partitions per sequence whose
+ * workgroups of 16 or 32 heads would leave half the CUs idle runs workgroups of 8 or 16 heads
+ * instead. Returns -1 on bad arguments
  * (num_kv_heads <= 0, num_heads not a positive multiple of it, kv_type not a kvb_kv_type). */
 int kvb_heads_per_workgroup(int num_heads, int num_kv_heads, int kv_type, int share_kv);
 

@@ -263,25 +263,35 @@ __device__ __forceinline__ int wave_inclusive_sum(int x) {
 // 512-token partitions, ran 124 us that way and 113 this way.)
 __device__ __forceinline__ WorkItem ragged_item(const int32_t* seq_lens, int batch, const SplitParams& sp, int len_cap,
                                                 int i, int items) {
-    const int part_tokens = sp.part_tokens;
-    // a sequence's full partitions
-    auto full = [&](int len) {
-        if (!sp.even) return fast_div(len, sp.part_div);
-        return len > 0 ? len / seq_part(sp, len) : 0;
-    };
     constexpr int E = kRaggedMaxBatch / 64;
     const int lane = threadIdx.x & 63;
     const int ne = (batch + 63) >> 6;
+    // every length in one round trip (a lane past the batch reads the last one): behind a branch per 64
+    // sequences each load was waited for in turn
     int len[E];
-    for (int e = 0; e < E; ++e) len[e] = (e < ne && 64 * e + lane < batch) ? live_len(seq_lens, 64 * e + lane, len_cap) : 0;
+    for (int e = 0; e < E; ++e) len[e] = seq_lens[min(64 * e + lane, batch - 1)];
+    // a sequence's full partitions, and the tokens of its partial last one
+    int full[E], rem[E];
+    for (int e = 0; e < E; ++e) {
+        full[e] = rem[e] = 0;
+        len[e] = 64 * e + lane < batch ? max(0, min(len[e], len_cap)) : 0;  // (live_len)
+        if (e >= ne) continue;  // uniform
+        if (sp.even) {
+            const int part = max(seq_part(sp, len[e]), 1);
+            full[e] = len[e] / part;
+            rem[e] = len[e] - full[e] * part;
+        } else {
+            full[e] = fast_div(len[e], sp.part_div);
+            rem[e] = len[e] - full[e] * sp.part_tokens;
+        }
+    }
     WorkItem r{-1, 0};
-    // full partitions, in sequence order: an exclusive scan of len / part_tokens
+    // full partitions, in sequence order: an exclusive scan of their counts
     int before = 0;
     for (int e = 0; e < E && e < ne; ++e) {
-        const int f = full(len[e]);
-        const int s = wave_inclusive_sum(f);
-        const int excl = before + s - f;
-        const unsigned long long hit = __ballot(f > 0 && excl <= i && i < excl + f);
+        const int s = wave_inclusive_sum(full[e]);
+        const int excl = before + s - full[e];
+        const unsigned long long hit = __ballot(full[e] > 0 && excl <= i && i < excl + full[e]);
         if (hit) {
             const int l = __ffsll(hit) - 1;
             r = WorkItem{64 * e + l, i - __builtin_amdgcn_readlane(excl, l)};
@@ -293,8 +303,7 @@ __device__ __forceinline__ WorkItem ragged_item(const int32_t* seq_lens, int bat
     int npart = 0, nempty = 0;
     unsigned key[E];
     for (int e = 0; e < E; ++e) {
-        const int rem = len[e] > 0 ? len[e] - full(len[e]) * seq_part(sp, len[e]) : 0;
-        key[e] = (e < ne && rem > 0) ? ((unsigned)rem << 16) | (0xFFFFu - (unsigned)(64 * e + lane)) : 0u;
+        key[e] = rem[e] > 0 ? ((unsigned)rem[e] << 16) | (0xFFFFu - (unsigned)(64 * e + lane)) : 0u;
         if (e < ne) {
             npart += __popcll(__ballot(key[e] != 0u));
             nempty += __popcll(__ballot(len[e] == 0 && 64 * e + lane < batch));
@@ -307,7 +316,7 @@ __device__ __forceinline__ WorkItem ragged_item(const int32_t* seq_lens, int bat
         int j = i - before;
         if (j < npart) {
             unsigned want = 0;
-            const int top = 16 + (32 - __builtin_clz((unsigned)part_tokens));  // keys < 2^top
+            const int top = 16 + (32 - __builtin_clz((unsigned)sp.part_tokens));  // keys < 2^top
             for (int bit = min(top, 32) - 1; bit >= 0; --bit) {
                 const unsigned cand = want | (1u << bit), hi = ~0u << bit;
                 int cnt = 0;
@@ -316,10 +325,10 @@ __device__ __forceinline__ WorkItem ragged_item(const int32_t* seq_lens, int bat
                 else j -= cnt;
             }
             const int b = 0xFFFF - (int)(want & 0xFFFFu);
-            int lb = 0;
+            int fb = 0;
             for (int e = 0; e < E && e < ne; ++e)
-                if (e == (b >> 6)) lb = __builtin_amdgcn_readlane(len[e], b & 63);
-            r = WorkItem{b, full(lb)};
+                if (e == (b >> 6)) fb = __builtin_amdgcn_readlane(full[e], b & 63);
+            r = WorkItem{b, fb};
         } else {
             // empty sequences, in sequence order
             int k = j - npart;

@@ -267,12 +267,30 @@ int ragged_items(const kvb_paged_args* a, const Split& sp) {
     return equal || items > 65535 ? 0 : (int)items;
 }
 
+// Query heads per workgroup of this step: kvb_heads_per_workgroup, but 8 (or 16 of 32) where the
+// workgroups of the wider kind would leave at least half the CUs idle. A KV head's workgroups then run on
+// CUs of their own (one XCD, so that the later reads of a page come from its L2), instead of as one
+// whose waves spend two or four heads' arithmetic per tile in turn; every head's sums are the same, to
+// fp32 rounding (16 of 32: to the bit). us, one 32- or 16-head workgroup / two or more: fp16 1 x 8192
+// tokens, one KV head, 512-token partitions, 32 heads 19.8 / 11.5, 16 heads 13.2 / 11.2; fp16 8 ragged up
+// to 8192, 2 KV heads, 32 heads 23.0 / 17.5; int8 2 x 2048, 8 KV heads, 16 heads 12.7 / 10.9. Past 16
+// partitions the wide workgroups keep their own merge.
+int step_heads(const kvb_paged_args* a, const Split& sp) {
+    const int qg = query_heads_per_group(a);
+    if (qg < 16 || sp.max_parts > 16) return qg;
+    long long items = 0;
+    for (int b = 0; b < a->batch; ++b) items += parts_of(a->host_seq_lens[b], sp);
+    for (const int few : {8, 16})
+        if (few < qg && 2 * items * (a->num_heads / (2 * few)) <= g.cus) return few;
+    return qg;
+}
+
 // counters: the fused merge's arrival counters (zero, at least B * H / qg ints), or null for the
 // library's own (grown on demand).
 int enqueue_paged(const kvb_paged_args* a, const Split& sp, float* part_out, float2* part_ml, bool fused,
                   const StepMarks& mk, bool loads_only = false, int* counters = nullptr) {
     const int part = sp.part;
-    const int qg = query_heads_per_group(a);
+    const int qg = step_heads(a, sp);
     kvbk::DecodeParams p{};
     p.q = a->q;
     p.k = a->k;

@@ -188,7 +188,7 @@ MUTANTS = [
     X("int8 q: second digit weighted 2^-6 instead of 2^-7",
       "const float wa = hl ? 1.0f / 128.0f : 1.0f,", "const float wa = hl ? 1.0f / 64.0f : 1.0f,"),
     X("int8 q: third digit dropped", "wb = hl ? 0.0f : 1.0f / 16384.0f;", "wb = 0.0f;"),
-    X("int8: K scale not applied", "if constexpr (KIND == KV_I8) f *= FAST ? ksh[h] : r.ks[j];", "(void)ksh;"),
+    X("int8: K scale not applied", "if constexpr (KIND == KV_I8) f *= FAST ? ksh[h] : kscale(j);", "(void)ksh;"),
     X("int8: scales of KV head 0 for every head (partition in lanes)",
       "const int soff = lane < nb ? (max(blkv, 0) * Hkv + kvh) * 4 : 0;",
       "const int soff = lane < nb ? (max(blkv, 0) * Hkv) * 4 : 0;"),
@@ -200,7 +200,7 @@ MUTANTS = [
       "float4 v = make_float4(a[0] + z[0], a[1] + z[1], a[2] + z[2], a[3] + z[3]);",
       "float4 v = make_float4(a[0], a[1], a[2], a[3]);"),
     X("int8: p * v_scale not normalised by the running power of two",
-      "(FAST ? vsh[j >> 2] : r.vs[j]) * vdown : 1.0f;", "(FAST ? vsh[j >> 2] : r.vs[j]) : 1.0f;"),
+      "(FAST ? vsh[j >> 2] : vscale(j)) * vdown : 1.0f;", "(FAST ? vsh[j >> 2] : vscale(j)) : 1.0f;"),
     X("int8: the V-scale power of two not undone at the end",
       "const float vupf = KIND == KV_I8 ? ldexpf(1.0f, ve) : 1.0f;", "const float vupf = 1.0f;"),
     X("tail mask off by one (the token at the partition end scored)",
@@ -225,7 +225,7 @@ MUTANTS = [
       "const float4 r = make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);",
       "const float4 r = make_float4(o.x, o.y, o.z, o.w);"),
     X("fused merge counts only the full partitions",
-      "const int nparts = (len + p.part_tokens - 1) / p.part_tokens;", "const int nparts = len / p.part_tokens;"),
+      "const int nparts = (len + PT - 1) / PT;", "const int nparts = len / PT;"),
     X("fused merge weighs every partition with partition 0's max",
       "add(o, L, partition_weight(ml[j].x, ml[j].y, M), pre[j]);",
       "add(o, L, partition_weight(ml[0].x, ml[j].y, M), pre[j]);"),
