@@ -153,7 +153,7 @@ struct CacheWriteArgs {
 double write_paged(const CacheWriteArgs&);
 
 // Each call queues the kernels on one stream, waits, and returns their GPU time in milliseconds,
-// from the first kernel's start to the last kernel's end (an event right before the first, one stamped by the last dispatch). Throws std::invalid_argument, before any GPU work, for a sequence length below
+// from the first kernel's start to the last kernel's end (events stamped by the dispatches). Throws std::invalid_argument, before any GPU work, for a sequence length below
 // 0, above max_len, or (paged) above max_blocks * page_size, and for the other refusals of
 // kvb_run_paged; std::runtime_error for device failures (src/metal_attn.hpp:82-87).
 double run_paged(const PagedArgs&);

@@ -211,12 +211,9 @@ struct NaiveParams {
     float2* stats;              // [B][H][chunks]: a chunk's (max score, exp-sum)
 };
 
-// Timing marks of a launch: `start` is recorded on the stream right before the kernel, `stop` is
-// stamped by the kernel's own dispatch with its end (the reference's GPUStartTime / GPUEndTime,
-// src/metal_attn.mm:119-130). Handing `start` to hipExtLaunchKernelGGL as well gave the same times
-// (10.6 us either way for a 10 us kernel on an idle stream, 11.7 either way right behind another
-// kernel) and cost 13 us of host time per launch: a waited-for 10 us kernel took 33.5 us that way,
-// 19.9 this way, and a queued one held the stream 5 us longer.
+// Timing marks of a launch: events that the kernel dispatch itself stamps with its start and end
+// (hipExtLaunchKernelGGL), so a pair brackets the kernels' execution and not the launch gap before
+// the first one (the reference's GPUStartTime / GPUEndTime, src/metal_attn.mm:119-130).
 struct Marks {
     hipEvent_t start = nullptr;
     hipEvent_t stop = nullptr;
@@ -229,10 +226,8 @@ struct Marks {
 template <typename... KArgs, typename... Args>
 inline void launch_marked_lds(void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t lds, hipStream_t s,
                               const Marks& m, Args... args) {
-    // (an error of the record is reported by the caller's hipGetLastError, like one of the launch)
-    if (m.start) (void)hipEventRecord(m.start, s);
-    if (m.stop)
-        hipExtLaunchKernelGGL(kernel, grid, block, lds, s, nullptr, m.stop, 0, args...);
+    if (m.start || m.stop)
+        hipExtLaunchKernelGGL(kernel, grid, block, lds, s, m.start, m.stop, 0, args...);
     else
         hipLaunchKernelGGL(kernel, grid, block, lds, s, args...);
 }
