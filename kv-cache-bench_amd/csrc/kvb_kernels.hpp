@@ -273,6 +273,10 @@ struct CacheWriteParams {
     int len_cap;                // live_len's cap: min(max_len, max_blocks * page_size)
     FastDiv page_div;           // division by page_size
     int row_shift;              // log2 of a row's 16-byte words (scatter)
+    int cus;                    // CUs of the device
+    int longest;                // the host's lengths: the largest,
+    long long live_tokens;      // their sum
+    long long live_blocks;      // (block, KV head) pairs that hold one of them
 };
 // grid (Hkv, batch, runs of tokens or groups of logical blocks): max_blocks_used = ceil(max_len / page)
 hipError_t launch_write_paged(const CacheWriteParams& p, int batch, int max_blocks_used, hipStream_t s,

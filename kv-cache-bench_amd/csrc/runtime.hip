@@ -892,6 +892,12 @@ int kvb_write_paged(const kvb_cache_args* a, double* ms) {
     p.page_div = kvbk::make_fast_div((uint32_t)a->page_size);
     while ((16 << p.row_shift) < p.head_dim * p.elem_size) ++p.row_shift;
     p.len_cap = (int)std::min((long long)a->max_len, (long long)a->max_blocks * a->page_size);
+    p.cus = g.cus;
+    for (int b = 0; b < a->batch; ++b) {
+        p.longest = std::max(p.longest, a->host_seq_lens[b]);
+        p.live_tokens += a->host_seq_lens[b];
+        p.live_blocks += ((long long)a->host_seq_lens[b] + a->page_size - 1) / a->page_size * a->num_kv_heads;
+    }
     hipEvent_t e0, e1;
     if (int st = get_event(&e0)) return st;
     if (int st = get_event(&e1)) return st;

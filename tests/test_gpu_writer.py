@@ -110,3 +110,28 @@ def test_writer_refusals_leave_the_pool(gpu):
     assert (paged.download(np.uint8, c.k.nbytes) == 0x33).all()
     for b in (contig, paged, table, lens):
         b.free()
+
+
+# Both sides of the lines between the quantiser's forms that the number of blocks draws (a wave per block
+# from 1024 blocks on, at the 256 CUs of an MI355X), and sequences that end long before their page does.
+@pytest.mark.parametrize("dim,page,batch,length", [(128, 16, 31, 256), (128, 16, 32, 256), (64, 32, 33, 511),
+                                                   (128, 1000, 2, 100), (64, 1000, 3, 300), (128, 200, 2, 230), (128, 140, 2, 129)])
+@pytest.mark.parametrize("max_len", [0, 700])
+def test_writer_block_counts(gpu, dim, page, batch, length, max_len):
+    kvb = gpu
+    lens = [length] * (batch - 1) + [length - 3]
+    w = kvb.Workload(kvb.Shape(batch, 4, 2, dim), "i8", lens, seed=page + batch, varied=True)
+    if max_len:  # a cache whose rows go on past the longest sequence
+        pad = [(0, 0), (0, 0), (0, max_len - length), (0, 0)]
+        w = kvb.Workload.from_arrays("i8", lens, w.q, np.pad(w.k, pad), np.pad(w.v, pad))
+    check_writer(kvb, w, page, page + 3, 1.2)
+
+
+@pytest.mark.parametrize("kv,batch", [("f16", 15), ("f16", 16), ("i8", 12), ("i8", 13)])
+def test_writer_full_size_streams(gpu, kv, batch):
+    """Calls either side of 128 MiB read and written, past which the rows are read with the streaming policy."""
+    kvb = gpu
+    per = 2048 * 8 * 128 * (4 if kv == "f16" else 5)
+    assert (batch * per >= 128 << 20) == ((kv, batch) in (("f16", 16), ("i8", 13)))
+    w = kvb.Workload(kvb.Shape(batch, 8, 8, 128), kv, [2048] * batch, seed=batch)
+    check_writer(kvb, w, 64, batch, 1.0)
