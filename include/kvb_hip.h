@@ -272,7 +272,7 @@ typedef struct kvb_naive_args {
     int kv_type;                 /* KVB_KV_F32 or KVB_KV_F16 */
     int max_len;                 /* row stride of the contiguous cache */
     const float* q;              /* device, float [B][H][D] */
-    const void* k;               /* device, kv_type [B][Hkv][max_len][D] */
+    const void* k;               /* device, kv_type [B][Hkv][max_len][D]; 16-byte aligned */
     const void* v;
     const int32_t* seq_lens;     /* device, int32 [B] */
     const int32_t* host_seq_lens;/* host copy of seq_lens */

@@ -107,6 +107,13 @@ __device__ __forceinline__ float wave_sum_f(float x) {
     return x;
 }
 
+// 16 bytes at any element's address: q and V are the caller's, aligned as their elements are. (The same
+// single 16-byte load: the unaligned ones of gfx950 need no other instruction.)
+typedef uint32_t u32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ uint4 load16(const void* p) {
+    return __builtin_bit_cast(uint4, *static_cast<const u32x4_any_t*>(p));
+}
+
 // Element e of a 16-byte word of f16 or f32 values.
 template <int KIND>
 __device__ __forceinline__ float word_at(const uint4& w, int e) {
@@ -143,7 +150,7 @@ __global__ __launch_bounds__(kNaiveThreads) void naive_scores_kernel(NaiveParams
         const int ng = min(kNaiveHeads, G - g0);
         __syncthreads();  // s_q and s_s of the previous heads are read
         for (int i = tid; i < ng * D / 4; i += kNaiveThreads)
-            reinterpret_cast<float4*>(&s_q[0][0])[i] = reinterpret_cast<const float4*>(p.q + (head0 + g0) * D)[i];
+            reinterpret_cast<uint4*>(&s_q[0][0])[i] = load16(p.q + (head0 + g0) * D + 4 * i);
         __syncthreads();
         for (int g = 0; g < ng; ++g) {
             float s[TW];
@@ -199,8 +206,7 @@ __global__ __launch_bounds__(kNaiveThreads) void naive_pv_kernel(NaiveParams p, 
     uint4 v[NL];
     for (int i = 0; i < NL; ++i) {
         const int t = min(t0 + wave * TW + i * RW + row, len - 1);  // (past the end: weight 0 below)
-        v[i] = *reinterpret_cast<const uint4*>(static_cast<const char*>(p.v) +
-                                               ((((size_t)b * p.num_kv_heads + kvh) * p.max_len + t) * VL + col) * 16);
+        v[i] = load16(static_cast<const char*>(p.v) + ((((size_t)b * p.num_kv_heads + kvh) * p.max_len + t) * VL + col) * 16);
     }
     const size_t head0 = (size_t)b * H + (size_t)kvh * G;
     for (int g0 = 0; g0 < G; g0 += NH) {
