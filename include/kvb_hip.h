@@ -279,7 +279,8 @@ typedef struct kvb_naive_args {
     float* out;                  /* device, float [B][H][D] */
 } kvb_naive_args;
 /* scores (with each 128-token chunk's softmax statistics) -> softmax and PV per chunk -> sum of the
- * chunks, with the scores in global memory. Refuses I8 and lengths < 0 or
+ * chunks, with the scores in global memory: a library scratch of B * H * max_len floats, max_len in whole
+ * chunks, and 8 bytes per chunk and head. Refuses I8 and lengths < 0 or
  * > max_len (src/metal_attn.mm:211-247). */
 int kvb_run_naive(const kvb_naive_args* a, double* ms);
 /* The refusals of kvb_run_naive alone. */

@@ -178,7 +178,7 @@ __global__ __launch_bounds__(kNaiveThreads) void naive_scores_kernel(NaiveParams
             if (in1) mx = fmaxf(mx, c);
             mx = wave_max_f(mx);
             const float sum = wave_sum_f((in0 ? __expf(a - mx) : 0.0f) + (in1 ? __expf(c - mx) : 0.0f));
-            float* dst = p.scores + h * p.max_len + t0;
+            float* dst = p.scores + (h * p.chunks + chunk) * C;
             if (in0) dst[lane] = a;
             if (in1) dst[64 + lane] = c;
             if (lane == 0) p.stats[h * p.chunks + chunk] = make_float2(mx, sum);
@@ -187,7 +187,8 @@ __global__ __launch_bounds__(kNaiveThreads) void naive_scores_kernel(NaiveParams
 }
 
 // Pass 2: the row's softmax (max and sum over its chunks' statistics), p_t = exp(s_t - max) / sum, and
-// part[b][h][chunk] = sum over the chunk of p_t v_t. Grid (chunks, Hkv, B). 16-byte words of V: VL
+// the chunk's share of the output, the sum over it of p_t v_t, which takes the place of its scores (no
+// other workgroup reads those). Grid (chunks, Hkv, B). 16-byte words of V: VL
 // lanes cover a row, a wave RW rows per load; all of a wave's rows are in flight at once, and each
 // lane keeps its PER columns of NH heads (1, 2, 4 or 8: with a run-time count the sums went to scratch
 // memory, 46 us against 8.9 at 2 x 4096 tokens).
@@ -225,7 +226,7 @@ __global__ __launch_bounds__(kNaiveThreads) void naive_pv_kernel(NaiveParams p, 
             float sum = 0.0f;
             for (int c = lane; c < nch; c += 64) sum += st[c].y * __expf(st[c].x - mx);
             const float inv = 1.0f / wave_sum_f(sum);
-            const float* sc = p.scores + h * p.max_len + t0;
+            const float* sc = p.scores + (h * p.chunks + chunk) * C;
             for (int t = lane; t < C; t += 64) s_p[g][t] = t0 + t < len ? __expf(sc[t] - mx) * inv : 0.0f;
         }
         __syncthreads();
@@ -256,7 +257,7 @@ __global__ __launch_bounds__(kNaiveThreads) void naive_pv_kernel(NaiveParams p, 
         for (int i = tid; i < ng * D; i += kNaiveThreads) {
             float a = 0.0f;
             for (int w = 0; w < W; ++w) a += s_o[w][i / D][i % D];
-            p.part[((head0 + g0 + i / D) * p.chunks + chunk) * D + i % D] = a;
+            p.scores[((head0 + g0 + i / D) * p.chunks + chunk) * C + i % D] = a;  // (its scores are in s_p)
         }
     }
 }
@@ -269,11 +270,11 @@ __global__ __launch_bounds__(D) void naive_sum_kernel(NaiveParams p) {
     const int h = blockIdx.x, b = blockIdx.y, d = threadIdx.x;
     const int nch = (live_len(p.seq_lens, b, p.max_len) + kNaiveChunk - 1) / kNaiveChunk;
     const size_t hb = (size_t)b * p.num_heads + h;
-    const float* src = p.part + hb * p.chunks * D + d;
+    const float* src = p.scores + hb * p.chunks * kNaiveChunk + d;
     float o = 0.0f;
     for (int c0 = 0; c0 < nch; c0 += U) {
         float x[U];
-        for (int j = 0; j < U; ++j) x[j] = src[(size_t)min(c0 + j, nch - 1) * D];
+        for (int j = 0; j < U; ++j) x[j] = src[(size_t)min(c0 + j, nch - 1) * kNaiveChunk];
         for (int j = 0; j < U; ++j) o += c0 + j < nch ? x[j] : 0.0f;
     }
     p.out[hb * D + d] = o;

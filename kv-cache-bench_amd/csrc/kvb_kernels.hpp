@@ -192,7 +192,8 @@ struct ReduceParams {
     int len_cap;                // as DecodeParams::len_cap
 };
 
-// Tokens one workgroup of the naive passes owns.
+// Tokens one workgroup of the naive passes owns: at least head_dim, whose share of the output it writes
+// over their scores.
 constexpr int kNaiveChunk = 128;
 
 struct NaiveParams {
@@ -200,14 +201,13 @@ struct NaiveParams {
     const void* k;              // [B][Hkv][max_len][D]
     const void* v;
     const int32_t* seq_lens;
-    float* scores;              // [B][H][max_len]
+    float* scores;              // [B][H][chunks][kNaiveChunk]: scores, then (head_dim of them) the chunk's share of the output
     float* out;
     int num_heads;
     int num_kv_heads;
     int max_len;
     float scale;
     int chunks;                 // max(1, ceil(max_len / kNaiveChunk))
-    float* part;                // [B][H][chunks][D]: a chunk's share of the output
     float2* stats;              // [B][H][chunks]: a chunk's (max score, exp-sum)
 };
 

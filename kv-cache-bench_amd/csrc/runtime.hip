@@ -913,7 +913,7 @@ int kvb_check_naive(const kvb_naive_args* a) {
     if (a->kv_type != KVB_KV_F32 && a->kv_type != KVB_KV_F16) return fail(KVB_EINVAL, "unknown kv_type");
     if (int st = check_shape(a->batch, a->num_heads, a->num_kv_heads, a->head_dim)) return st;
     if (a->max_len < 0) return fail(KVB_EINVAL, "max_len < 0");
-    // launch grids (max_len / 16, H, batch) and (H, batch): y and z are at most 65535
+    // launch grids (chunks, Hkv, batch) and (H, batch): y and z are at most 65535
     if (a->batch > 65535 || a->num_heads > 65535) return fail(KVB_EINVAL, "batch or num_heads > 65535");
     if (a->batch > 0 && !a->host_seq_lens) return fail(KVB_EINVAL, "host_seq_lens is required");
     if (int st = check_lens(a->batch, a->host_seq_lens, a->max_len, (size_t)a->max_len)) return st;
@@ -927,17 +927,15 @@ int kvb_run_naive(const kvb_naive_args* a, double* ms) {
     if (int st = kvb_check_naive(a)) return st;
     if (int st = ensure_device()) return st;
     if (a->batch == 0) return KVB_OK;
-    // scores [rows][max_len], then each chunk's parts of the output and (max, sum), 16-byte aligned
+    // a row's scores in whole chunks, each then its share of the output; then each chunk's (max, sum)
     const size_t rows = (size_t)a->batch * a->num_heads;
     const size_t chunks = ((size_t)std::max(a->max_len, 1) + kvbk::kNaiveChunk - 1) / kvbk::kNaiveChunk;
-    const size_t score_floats = (rows * (size_t)std::max(a->max_len, 1) + 3) / 4 * 4;
-    const size_t part_floats = rows * chunks * (size_t)a->head_dim;
-    const size_t need = (score_floats + part_floats + 2 * rows * chunks) * sizeof(float);
-    if (int st = grow(&g.scores, &g.scores_bytes, need)) return st;
+    const size_t score_floats = rows * chunks * kvbk::kNaiveChunk;
+    if (int st = grow(&g.scores, &g.scores_bytes, (score_floats + 2 * rows * chunks) * sizeof(float))) return st;
     float* scores = static_cast<float*>(g.scores);
     kvbk::NaiveParams p{a->q, a->k, a->v, a->seq_lens, scores, a->out, a->num_heads, a->num_kv_heads, a->max_len,
-                        1.0f / std::sqrt((float)a->head_dim), (int)chunks, scores + score_floats,
-                        reinterpret_cast<float2*>(scores + score_floats + part_floats)};
+                        1.0f / std::sqrt((float)a->head_dim), (int)chunks,
+                        reinterpret_cast<float2*>(scores + score_floats)};
     hipEvent_t e0, e1;
     if (int st = get_event(&e0)) return st;
     if (int st = get_event(&e1)) return st;
@@ -953,8 +951,7 @@ int kvb_run_attention_fp64(const kvb_naive_args* a, double* ms) {
     if (int st = ensure_device()) return st;
     if (a->batch == 0) return KVB_OK;
     kvbk::NaiveParams p{a->q, a->k, a->v, a->seq_lens, nullptr, a->out,
-                        a->num_heads, a->num_kv_heads, a->max_len, 1.0f / std::sqrt((float)a->head_dim), 0, nullptr,
-                        nullptr};
+                        a->num_heads, a->num_kv_heads, a->max_len, 1.0f / std::sqrt((float)a->head_dim), 0, nullptr};
     hipEvent_t e0, e1;
     if (int st = get_event(&e0)) return st;
     if (int st = get_event(&e1)) return st;

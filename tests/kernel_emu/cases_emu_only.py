@@ -15,7 +15,11 @@ every access inside the buffers. On top of that:
 Reference: the reference's kernel reads seq_lens as given (src/kernels.metal:44-47) and its host
 refuses lengths past the capacity (src/metal_attn.mm:107-117); the output for lengths that disagree
 is unspecified in both.
+
+The emulation counts device memory, too: what a call keeps allocated is checked here.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -104,3 +108,24 @@ def test_graph_replay_with_device_lengths_that_disagree(emu, kv):
             if graph is not None:
                 graph.free()
             dev.free()
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+def test_naive_scratch_holds_the_scores_and_little_more(emu, dim):
+    """The baseline's scratch is B * H * max_len floats, in whole 128-token chunks, and two floats a chunk."""
+    kvb = emu
+    max_len, heads = 24000 + dim, 32
+    shape = kvb.Shape(2, heads, 1, dim)
+    rng = np.random.default_rng(dim)
+    kv = rng.random((2, 1, max_len, dim), np.float32)
+    w = kvb.Workload.from_arrays("f32", [3, 1], rng.random((2, heads, dim), np.float32), kv, kv)
+    bufs = [kvb.Buffer.from_array(x) for x in (w.q, w.k, w.v, w.lens)]
+    out = kvb.Buffer(w.out_floats() * 4)
+    kvb.hip.kvbemu_device_bytes.restype = ctypes.c_size_t
+    before = kvb.hip.kvbemu_device_bytes()
+    kvb.run_naive(w, out, *bufs)
+    scores = shape.batch * heads * max_len * 4
+    assert kvb.hip.kvbemu_device_bytes() - before <= scores * 1.03
+    for b in bufs:
+        b.free()
+    out.free()

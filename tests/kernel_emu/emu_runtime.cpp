@@ -345,6 +345,12 @@ void record(hipEvent_t e) {
 }  // namespace kvbemu
 
 extern "C" const char* kvbemu_last_error(void) { return kvbemu::g_last_msg.c_str(); }
+// Device memory allocated and not freed, the registered symbols included.
+extern "C" size_t kvbemu_device_bytes(void) {
+    size_t n = 0;
+    for (const auto& [base, bytes] : kvbemu::g_allocs) n += bytes;
+    return n;
+}
 
 const char* hipGetErrorString(hipError_t e) {
     switch (e) {
