@@ -415,6 +415,7 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
     // groups of 16: 163.5 -> 106.9 us fp16, 88.2 -> 68.0 int8, against 133.7 / 80.9 with the sibling
     // order alone; non-temporal stays for one workgroup per KV head: 84.5 us there, 93.9 without).
     // Head splits (HS > 1) read each tile once per split: ordinary loads, as SHARE (SHL: once).
+    // (On the any-page path the host picks SHARE for other reasons, too: DecodeParams::share_pages.)
     constexpr int kKvPolicy = SHARE || (HS > 1 && !SHL) ? 0 : kNonTemporal;
 
     // Per wave: the V tile (32 rows of D elements, swizzled); after the loop it holds the wave's
@@ -1573,16 +1574,24 @@ hipError_t launch_one(const DecodeParams& p, int batch, hipStream_t s, const Mar
     return hipGetLastError();
 }
 
+// Any page size: the build that stages the blocks the launch's workgroups touch.
+template <int KIND, int D, int QG, bool PART, bool SHARE>
+hipError_t launch_any_page(const DecodeParams& p, int batch, hipStream_t s, const Marks& m) {
+    if constexpr (KIND != KV_F16)
+        if (p.table_in_lds && p.table_in_lds <= kTableStageSmall)
+            return launch_one<KIND, D, QG, false, false, PART, SHARE, kTableStageSmall>(p, batch, s, m);
+    return p.table_in_lds ? launch_one<KIND, D, QG, false, false, PART, SHARE, kTableStage>(p, batch, s, m)
+                          : launch_one<KIND, D, QG, false, false, PART, SHARE>(p, batch, s, m);
+}
+
 // Two partitions per workgroup (DecodeParams::pair): tile-aligned f16 and i8 caches, plain grid only.
+// SHARE: of the tile-aligned build (the host picks the any-page one's).
 template <int KIND, int D, int QG, bool PART, bool SHARE = false>
 hipError_t launch_qg(bool fast, const DecodeParams& p, int batch, hipStream_t s, const Marks& m) {
     if (!fast) {
         if (p.pair) return hipErrorInvalidValue;
-        if constexpr (KIND != KV_F16)
-            if (p.table_in_lds && p.table_in_lds <= kTableStageSmall)
-                return launch_one<KIND, D, QG, false, false, PART, SHARE, kTableStageSmall>(p, batch, s, m);
-        return p.table_in_lds ? launch_one<KIND, D, QG, false, false, PART, SHARE, kTableStage>(p, batch, s, m)
-                              : launch_one<KIND, D, QG, false, false, PART, SHARE>(p, batch, s, m);
+        return p.share_pages ? launch_any_page<KIND, D, QG, PART, true>(p, batch, s, m)
+                             : launch_any_page<KIND, D, QG, PART, false>(p, batch, s, m);
     }
     if constexpr (KIND != KV_F32 && decode_shape(KIND, QG).hs == 1) {
         if (p.pair) return p.ragged_items ? hipErrorInvalidValue : launch_one<KIND, D, QG, true, true, PART, SHARE>(p, batch, s, m);
@@ -1596,9 +1605,10 @@ template <int KIND, int D>
 hipError_t launch_for_dim(int qg, bool fast, const DecodeParams& p, int batch, hipStream_t s, const Marks& m) {
     const bool sib = p.group > qg;  // more than one workgroup per KV head
     switch (qg) {
-        // SHARE builds where a KV head has more than one workgroup and one workgroup serves 3 or 5-8
-        // heads (groups 9, 10, 12, 14, 16, 24, 32, ...); groups whose workgroups serve 1, 2 or 4
-        // heads each (11, 13, 22, 44, ...) keep the plain order and non-temporal loads.
+        // Tile-aligned pages: SHARE builds where a KV head has more than one workgroup and one workgroup
+        // serves 3 or 5-8 heads (groups 9, 10, 12, 14, 16, 24, 32, ...); groups whose workgroups serve 1,
+        // 2 or 4 heads each (11, 13, 22, 44, ..., and share_kv 0) keep the plain order and non-temporal
+        // loads.
         case 1: return launch_qg<KIND, D, 1, false>(fast, p, batch, s, m);
         case 2: return launch_qg<KIND, D, 2, false>(fast, p, batch, s, m);
         case 3: return sib ? launch_qg<KIND, D, 4, true, true>(fast, p, batch, s, m)

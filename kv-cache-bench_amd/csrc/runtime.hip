@@ -285,6 +285,25 @@ int step_heads(const kvb_paged_args* a, const Split& sp) {
     return qg;
 }
 
+// The any-page path's SHARE build: ordinary loads, and the workgroups of one KV head side by side on one
+// XCD. Where a KV head has several workgroups they read the same rows, and the later ones find them in
+// that XCD's L2 (us, this / the plain order with non-temporal loads, page 24: fp16, 8 x 16384 tokens, group
+// 22, 125 / 254; 16 x 4096, 8 KV heads, one head per workgroup, 116 / 191; fp32, 8 x 16384, 919 / 1406). int8
+// in workgroups of 1, 2 or 4 heads only from 32 MB of cache on (8 x 16384, group 22, 111 / 141; 22 ragged
+// up to 183, one head per workgroup, page 8, 20.5 / 17.2). With one workgroup per KV head it is the loads that
+// matter: a cache that the 256 MiB memory-side cache holds is best read with ordinary ones (fp16, repeated and
+// after a flush: 20 ragged up to 2313, page 1, 25.4 / 29.6 and 30.3 / 32.5; 16 x 4096, 8 KV heads, 268 MB,
+// 45.9 / 52.5 and 58.8 / 55.4), a larger one with non-temporal ones (8 x 16384, 537 MB, 100 / 90 and 100 / 93).
+// int8 is the faster with non-temporal ones at every size, by 2-6%.
+bool share_pages(const kvb_paged_args* a, int qg) {
+    long long bytes = 0;
+    for (int b = 0; b < a->batch; ++b) bytes += a->host_seq_lens[b];
+    bytes *= 2LL * a->num_kv_heads * a->head_dim * (a->kv_type == KVB_KV_F32 ? 4 : a->kv_type == KVB_KV_F16 ? 2 : 1);
+    const bool siblings = a->num_heads / a->num_kv_heads > qg, few = qg == 1 || qg == 2 || qg == 4;
+    if (a->kv_type == KVB_KV_I8) return siblings && (!few || bytes >= 32LL << 20);
+    return siblings || bytes <= 256LL << 20;
+}
+
 // counters: the fused merge's arrival counters (zero, at least B * H / qg ints), or null for the
 // library's own (grown on demand).
 int enqueue_paged(const kvb_paged_args* a, const Split& sp, float* part_out, float2* part_ml, bool fused,
@@ -346,6 +365,7 @@ int enqueue_paged(const kvb_paged_args* a, const Split& sp, float* part_out, flo
     p.table_in_lanes = fast && nb_max <= kvbk::kLaneBlocks;
     p.table_in_lds = !fast && nb_max <= kvbk::kTableStage ? (int)nb_max : 0;
     p.quads = a->page_size % 4 == 0 && part % 4 == 0;
+    if (!fast) p.share_pages = share_pages(a, qg);
     const kvbk::Marks dm{mk.step.start ? mk.step.start : mk.decode.start, fused ? mk.step.stop : mk.decode.stop,
                          mk.step.describe, mk.step.describe_cap};
     const kvbk::Marks rm{mk.reduce.start, mk.step.stop ? mk.step.stop : mk.reduce.stop};
