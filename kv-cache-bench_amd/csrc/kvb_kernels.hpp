@@ -148,6 +148,7 @@ struct DecodeParams {
     int quads;                  // page_size and the partition are multiples of 4: 4 aligned tokens share a page
     SplitParams split;          // split.part_tokens == part_tokens
     int share_pages;            // any-page path: the SHARE build
+    int refill;                 // fp32: the REFILL build
 };
 
 // Block ids the any-page kernel stages in LDS per workgroup (16 KB): a 4096-token partition at any

@@ -351,7 +351,9 @@ __device__ __forceinline__ WorkItem ragged_item(const int32_t* seq_lens, int bat
 // lane. The tile-aligned int8 kernel is held to 3 (168 VGPRs, no spills), so that three of its
 // workgroups share a CU on multi-round grids; at 169 VGPRs it would drop to two. With one query head
 // per workgroup it would spill there, so that case keeps 2, as do the PAIR kernels, which run one
-// workgroup per CU.)
+// workgroup per CU. fp32 at head_dim 64 without REFILL fits 4 on tile-aligned pages (fp32, 4 x 8192 tokens,
+// group 64: 28.9 us with 4 workgroups per CU, 33.9 with 3); REFILL at head_dim 128 runs one workgroup per
+// CU by its rule, and would spill with 256 registers.)
 // LOADS: the measurement variant (kvb_run_paged_loads). It issues every load of the decode in the
 // same order and consumes the registers with XORs, and computes and writes nothing.
 // PAIR: a workgroup computes two consecutive partitions (grid z = ceil(max_parts / 2)), so that a grid
@@ -363,11 +365,14 @@ __device__ __forceinline__ WorkItem ragged_item(const int32_t* seq_lens, int bat
 // HS head splits of TS token streams): a wave walks its stream's tiles for its split's heads. int8:
 // each tile is read by HS waves, the first from HBM and the others mostly from the CU's caches, with
 // ordinary loads; fp16: the stream's two waves load half a tile each and share it through LDS (SHL).
+// REFILL (fp32): the next tile's loads go out as the present one is used (see the tile walk).
 template <int KIND, int D, int QG, bool FAST, bool LOADS = false, bool PAIR = false, bool PART = false,
-          bool SHARE = false, int STAGE = 0>
+          bool SHARE = false, int STAGE = 0, bool REFILL = false>
 __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdgpu_waves_per_eu(
     decode_wg_waves(KIND, QG) > 4 ? 2
     : decode_shape(KIND, QG).qw > 8 ? 1
+    : KIND == KV_F32 && FAST && D == 64 && !REFILL ? 4
+    : REFILL && D == 128 ? 1
     : KIND == KV_I8 && FAST && !LOADS && !PAIR && QG > 1 ? 3 : 2))) void paged_decode_kernel(DecodeParams p) {
     using T = KvT<KIND, D>;
     using R = TileRegs<KIND, D>;
@@ -771,7 +776,7 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
             __builtin_amdgcn_sched_barrier(0);
         }
     } else {
-        for (int k = 0; k + 1 < NBUF || k == 0; ++k) {
+        for (int k = 0; k + 1 < NBUF || (REFILL && k == 0); ++k) {
             load_tile(r[k], t0 + (it + k * TS) * kTok);
             // (in buffer order, as the loop issues them: the loop head is entered from here and from the
             // back edge, and the wait for buffer 0 there can leave the later buffers in flight only if
@@ -1223,7 +1228,7 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
 #pragma unroll
         for (int k = 0; k < NBUF; ++k) {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // tile `it` (buffer k) has arrived
-            if constexpr (NBUF > 1) {
+            if constexpr (!REFILL) {
                 load_tile(r[(k + NBUF - 1) % NBUF], t0 + (it + (NBUF - 1) * TS) * kTok);
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -1247,6 +1252,8 @@ __global__ __launch_bounds__(64 * decode_wg_waves(KIND, QG)) __attribute__((amdg
                 // head_dim 128 keeps it: the branch cost its long walks 3-6% (16 x 8192 tokens 43.8 -> 46.7
                 // us), more than the step costs its short ones.
                 if (k == 0 || (KIND == KV_I8 && FAST && D == 128) || it < ntiles) compute_tile(r[k], t0 + it * kTok, [] {}, [] {});
+            } else if constexpr (!REFILL) {
+                compute_tile(r[0], t0 + it * kTok, [] {}, [] {});
             } else {
                 // fp32: one buffer, refilled with the next tile as it is used: V's registers once the V
                 // rows are in LDS, K's once the scores are computed. (Any page: without the branch past
@@ -1547,14 +1554,14 @@ hipError_t loads_only_lds(size_t* lds) {
     return hipSuccess;
 }
 
-template <int KIND, int D, int QG, bool FAST, bool PAIR, bool PART, bool SHARE, int STAGE = 0>
+template <int KIND, int D, int QG, bool FAST, bool PAIR, bool PART, bool SHARE, int STAGE = 0, bool REFILL = false>
 hipError_t launch_one(const DecodeParams& p, int batch, hipStream_t s, const Marks& m) {
     if (m.describe) {  // the demangled name of the instantiation below, as rocprofv3 prints it
         auto tf = [](bool x) { return x ? "true" : "false"; };
         const bool loads = FAST && p.loads_only;
         std::snprintf(m.describe, m.describe_cap,
-                      "void kvbk::paged_decode_kernel<%d, %d, %d, %s, %s, %s, %s, %s, %d>(kvbk::DecodeParams)", KIND, D,
-                      QG, tf(FAST), tf(loads), tf(PAIR), tf(PART), tf(SHARE), loads ? 0 : STAGE);
+                      "void kvbk::paged_decode_kernel<%d, %d, %d, %s, %s, %s, %s, %s, %d, %s>(kvbk::DecodeParams)", KIND, D,
+                      QG, tf(FAST), tf(loads), tf(PAIR), tf(PART), tf(SHARE), loads ? 0 : STAGE, tf(!loads && REFILL));
         return hipSuccess;
     }
     const int gz = PAIR ? (p.max_parts + 1) / 2 : p.max_parts;
@@ -1569,9 +1576,17 @@ hipError_t launch_one(const DecodeParams& p, int batch, hipStream_t s, const Mar
                               lds, s, m, p);
         }
     } else {
-        launch_marked(paged_decode_kernel<KIND, D, QG, FAST, false, PAIR, PART, SHARE, STAGE>, grid, dim3(64 * decode_wg_waves(KIND, QG)), s, m, p);
+        launch_marked(paged_decode_kernel<KIND, D, QG, FAST, false, PAIR, PART, SHARE, STAGE, REFILL>, grid, dim3(64 * decode_wg_waves(KIND, QG)), s, m, p);
     }
     return hipGetLastError();
+}
+
+// fp32: the REFILL build where the host asks for it.
+template <int KIND, int D, int QG, bool FAST, bool PART, bool SHARE, int STAGE>
+hipError_t launch_walk(const DecodeParams& p, int batch, hipStream_t s, const Marks& m) {
+    if constexpr (KIND == KV_F32)
+        if (p.refill) return launch_one<KIND, D, QG, FAST, false, PART, SHARE, STAGE, true>(p, batch, s, m);
+    return launch_one<KIND, D, QG, FAST, false, PART, SHARE, STAGE>(p, batch, s, m);
 }
 
 // Any page size: the build that stages the blocks the launch's workgroups touch.
@@ -1579,9 +1594,9 @@ template <int KIND, int D, int QG, bool PART, bool SHARE>
 hipError_t launch_any_page(const DecodeParams& p, int batch, hipStream_t s, const Marks& m) {
     if constexpr (KIND != KV_F16)
         if (p.table_in_lds && p.table_in_lds <= kTableStageSmall)
-            return launch_one<KIND, D, QG, false, false, PART, SHARE, kTableStageSmall>(p, batch, s, m);
-    return p.table_in_lds ? launch_one<KIND, D, QG, false, false, PART, SHARE, kTableStage>(p, batch, s, m)
-                          : launch_one<KIND, D, QG, false, false, PART, SHARE>(p, batch, s, m);
+            return launch_walk<KIND, D, QG, false, PART, SHARE, kTableStageSmall>(p, batch, s, m);
+    return p.table_in_lds ? launch_walk<KIND, D, QG, false, PART, SHARE, kTableStage>(p, batch, s, m)
+                          : launch_walk<KIND, D, QG, false, PART, SHARE, 0>(p, batch, s, m);
 }
 
 // Two partitions per workgroup (DecodeParams::pair): tile-aligned f16 and i8 caches, plain grid only.
@@ -1598,7 +1613,7 @@ hipError_t launch_qg(bool fast, const DecodeParams& p, int batch, hipStream_t s,
     } else {
         if (p.pair) return hipErrorInvalidValue;
     }
-    return launch_one<KIND, D, QG, true, false, PART, SHARE>(p, batch, s, m);
+    return launch_walk<KIND, D, QG, true, PART, SHARE, 0>(p, batch, s, m);
 }
 
 template <int KIND, int D>

@@ -252,6 +252,13 @@ long long parts_of(int len, const Split& sp) {
     return (len + part - 1) / part;
 }
 
+// Workgroups of a step that hold tokens.
+long long workgroups(const kvb_paged_args* a, const Split& sp, int qg) {
+    long long items = 0;
+    for (int b = 0; b < a->batch; ++b) items += parts_of(a->host_seq_lens[b], sp);
+    return items * (a->num_heads / qg);
+}
+
 // Work items of a ragged batch in the kernel's longest-first order (one per partition holding
 // tokens, one per empty sequence), or 0 for the plain (sequence, partition) grid: sequences of equal
 // length gain nothing from reordering, and the order needs one lane per sequence.
@@ -278,10 +285,8 @@ int ragged_items(const kvb_paged_args* a, const Split& sp) {
 int step_heads(const kvb_paged_args* a, const Split& sp) {
     const int qg = query_heads_per_group(a);
     if (qg < 16 || sp.max_parts > 16) return qg;
-    long long items = 0;
-    for (int b = 0; b < a->batch; ++b) items += parts_of(a->host_seq_lens[b], sp);
     for (const int few : {8, 16})
-        if (few < qg && 2 * items * (a->num_heads / (2 * few)) <= g.cus) return few;
+        if (few < qg && 2 * workgroups(a, sp, 2 * few) <= g.cus) return few;
     return qg;
 }
 
@@ -366,6 +371,12 @@ int enqueue_paged(const kvb_paged_args* a, const Split& sp, float* part_out, flo
     p.table_in_lds = !fast && nb_max <= kvbk::kTableStage ? (int)nb_max : 0;
     p.quads = a->page_size % 4 == 0 && part % 4 == 0;
     if (!fast) p.share_pages = share_pages(a, qg);
+    // fp32's next tile under the present one (REFILL): where a workgroup has its CU to itself, so that
+    // nothing else covers its loads, and a wave has a second tile. (Against the walk that loads a tile when
+    // it needs it, times over shapes of 4 tiles a wave and more: 0.89-0.97 at one workgroup per CU, 1.00 at
+    // two and more, up to 1.2 where siblings read the pages through L2; single tiles lose a round trip on the
+    // refill: page 2, 89 tokens, 14 sequences 9.5 / 11.5 us.)
+    p.refill = a->kv_type == KVB_KV_F32 && part >= 2 * kvbk::kEvenTokens && workgroups(a, sp, qg) <= g.cus;
     const kvbk::Marks dm{mk.step.start ? mk.step.start : mk.decode.start, fused ? mk.step.stop : mk.decode.stop,
                          mk.step.describe, mk.step.describe_cap};
     const kvbk::Marks rm{mk.reduce.start, mk.step.stop ? mk.step.stop : mk.reduce.stop};

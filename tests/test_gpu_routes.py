@@ -10,7 +10,7 @@ from conftest import progress
 
 pytestmark = pytest.mark.gpu
 
-FIELDS = ("kind", "dim", "heads", "fast", "loads", "pair", "part", "share", "stage")
+FIELDS = ("kind", "dim", "heads", "fast", "loads", "pair", "part", "share", "stage", "refill")
 
 
 def build_of(kvb, dev, part, share_kv=True):
@@ -86,4 +86,23 @@ def test_large_caches_are_read_with_streaming_loads(gpu):
         a.max_len, a.max_blocks, a.host_seq_lens = n, n // 24 + 1, lens.ctypes.data
         kvb.check(kvb.hip.kvb_paged_kernel_name(ctypes.byref(a), 0, buf, 512), "paged_kernel_name")
         assert buf.value.decode().split("<")[1].split(">")[0].split(", ")[7] == share
+    dev.free()
+
+
+@pytest.mark.parametrize("heads", [(8, 2, 64), (8, 2, 128), (24, 2, 64), (12, 2, 128)])
+@pytest.mark.parametrize("page", [16, 24])
+@pytest.mark.parametrize("lens,part", [([1000, 600], 256), ([1000, 600], 128), ([257] * 2, 300), ([300] * 64, 256),
+                                       ([300] * 65, 256), ([300] * 32, 256), ([300] * 33, 256)])
+def test_fp32_refills_where_a_workgroup_has_its_cu(gpu, oracle, heads, page, lens, part):
+    """The build that loads the next tile under the present one: at most one workgroup per CU (of 256), and
+    two tiles a wave."""
+    kvb = gpu
+    w = kvb.Workload(kvb.Shape(len(lens), *heads), "f32", lens, seed=page + part)
+    c = kvb.PagedCache(w, page, part, pool_factor=1.1, poison=True)
+    dev = kvb.DeviceCase(w, c)
+    groups = heads[0] // kvb.heads_per_workgroup(w.shape, kvb.KV_F32) * sum(-(-n // part) for n in lens)
+    assert build_of(kvb, dev, part)["refill"] == ("true" if part >= 256 and groups <= 256 else "false")
+    dev.out.fill(0xFF)
+    dev.run(part)
+    pb.check_output(kvb, oracle, w, c, dev.output())
     dev.free()
