@@ -280,13 +280,17 @@ int ragged_items(const kvb_paged_args* a, const Split& sp) {
 // whose waves spend two or four heads' arithmetic per tile in turn; every head's sums are the same, to
 // fp32 rounding (16 of 32: to the bit). us, one 32- or 16-head workgroup / two or more: fp16 1 x 8192
 // tokens, one KV head, 512-token partitions, 32 heads 19.8 / 11.5, 16 heads 13.2 / 11.2; fp16 8 ragged up
-// to 8192, 2 KV heads, 32 heads 23.0 / 17.5; int8 2 x 2048, 8 KV heads, 16 heads 12.7 / 10.9. Past 16
-// partitions the wide workgroups keep their own merge.
+// to 8192, 2 KV heads, 32 heads 23.0 / 17.5; int8 2 x 2048, 8 KV heads, 16 heads 12.7 / 10.9; 1 x 65536
+// tokens, 8 KV heads, 4096-token partitions, 16 heads, fp16 71.1 / 47.8, int8 43.6 / 41.4. int8 at head_dim
+// 64, whose 16-head tile is the cheapest, gains from workgroups of 8 only where seven CUs of eight would
+// idle: 1 x 8192, one KV head, 10.0 / 9.5, but 4 x 16384, 2 KV heads, 1024-token partitions, 14.5 / 15.7.
+// Past 16 partitions the wide workgroups keep their own merge.
 int step_heads(const kvb_paged_args* a, const Split& sp) {
     const int qg = query_heads_per_group(a);
     if (qg < 16 || sp.max_parts > 16) return qg;
+    const int share = a->kv_type == KVB_KV_I8 && a->head_dim == 64 && qg == 16 ? 8 : 2;  // of the CUs
     for (const int few : {8, 16})
-        if (few < qg && 2 * workgroups(a, sp, 2 * few) <= g.cus) return few;
+        if (few < qg && share * workgroups(a, sp, 2 * few) <= g.cus) return few;
     return qg;
 }
 

@@ -106,3 +106,19 @@ def test_fp32_refills_where_a_workgroup_has_its_cu(gpu, oracle, heads, page, len
     dev.run(part)
     pb.check_output(kvb, oracle, w, c, dev.output())
     dev.free()
+
+
+# kv, group, head_dim, sequences of 1000 tokens with 4 partitions each, heads per workgroup: the wide
+# workgroups where they fill half the CUs (of 256), int8 groups of 16 at head_dim 64 an eighth of them
+@pytest.mark.parametrize("kv,group,dim,batch,heads", [
+    ("f16", 16, 64, 32, 8), ("f16", 16, 64, 33, 16), ("i8", 16, 128, 32, 8), ("i8", 16, 128, 33, 16),
+    ("i8", 16, 64, 8, 8), ("i8", 16, 64, 9, 16), ("i8", 16, 64, 33, 16),
+    ("i8", 32, 64, 16, 8), ("i8", 32, 64, 17, 16), ("i8", 32, 64, 32, 16), ("i8", 32, 64, 33, 32),
+])
+def test_wide_groups_on_few_workgroups(gpu, kv, group, dim, batch, heads):
+    kvb = gpu
+    w = kvb.Workload(kvb.Shape(batch, group, 1, dim), kv, [1000] * batch, seed=batch)
+    c = kvb.PagedCache(w, 64, 1)
+    dev = kvb.DeviceCase(w, c)
+    assert build_of(kvb, dev, 256)["heads"] == str(heads)
+    dev.free()
