@@ -120,6 +120,10 @@ int kvb_auto_part_tokens(int batch, int num_kv_heads, int max_len);
 /* Partitions per (sequence, head) in the workspace: max(1, ceil(max_len / part)) with part
  * resolved as kvb_run_paged does (src/metal_attn.mm:160-161). Returns -1 on bad arguments. */
 int kvb_paged_max_parts(const kvb_paged_args* a);
+/* Not in the reference: tokens per partition of kvb_run_paged's step with these arguments; at part_tokens 0
+ * without a workspace, the most that one of the library's even cut holds. Same refusals as kvb_run_paged
+ * (-1, kvb_last_error); launches nothing. */
+int kvb_paged_part_tokens(const kvb_paged_args* a);
 /* Bytes of the workspace a call with these arguments uses (0 on bad arguments). */
 size_t kvb_paged_workspace_bytes(const kvb_paged_args* a);
 /* Query heads one paged_decode workgroup serves, which read each K/V page once together: with

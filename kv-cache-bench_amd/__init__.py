@@ -95,6 +95,7 @@ _SIGS = {
     "kvb_auto_part_tokens": ([_i, _i, _i], _i),
     "kvb_heads_per_workgroup": ([_i, _i, _i, _i], _i),
     "kvb_paged_max_parts": ([_PA], _i),
+    "kvb_paged_part_tokens": ([_PA], _i),
     "kvb_paged_workspace_bytes": ([_PA], _sz),
     "kvb_check_paged": ([_PA], _i),
     "kvb_run_paged": ([_PA, _d], _i),
@@ -487,6 +488,14 @@ class DeviceCase:
     def max_parts(self, part_tokens=0):
         a = self.args(part_tokens)
         return hip.kvb_paged_max_parts(ctypes.byref(a))
+
+    def part_tokens(self, part_tokens=0):
+        """Tokens per partition of the step run() runs (kvb_paged_part_tokens)."""
+        a = self.args(part_tokens)
+        part = hip.kvb_paged_part_tokens(ctypes.byref(a))
+        if part < 0:
+            raise KvbInvalidArgument(f"paged_part_tokens: {hip.kvb_last_error().decode()}")
+        return part
 
     def free(self):
         for b in (self.q, self.k, self.v, self.table, self.lens, self.k_scale, self.v_scale, self.out):

@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <cstring>
 #include <iterator>
+#include <numeric>
 #include <string>
 #include <utility>
 #include <vector>
@@ -370,7 +371,10 @@ int enqueue_paged(const kvb_paged_args* a, const Split& sp, float* part_out, flo
     // blocks one workgroup's range touches: its tokens / page when the page divides them (the range
     // then starts on a page), else at most two more
     const long long span = (p.pair ? 2LL : 1LL) * part;
-    const long long nb_max = span % a->page_size == 0 ? span / a->page_size : span / a->page_size + 2;
+    long long nb_max = span % a->page_size == 0 ? span / a->page_size : span / a->page_size + 2;
+    // (an even split's shorter partitions, at least kEvenTokens less, start on any multiple of kEvenTokens)
+    if (sp.even && part > kvbk::kEvenTokens)
+        nb_max = std::max(nb_max, (2LL * a->page_size - std::gcd(a->page_size, kvbk::kEvenTokens) + part - kvbk::kEvenTokens - 1) / a->page_size);
     p.table_in_lanes = fast && nb_max <= kvbk::kLaneBlocks;
     p.table_in_lds = !fast && nb_max <= kvbk::kTableStage ? (int)nb_max : 0;
     p.quads = a->page_size % 4 == 0 && part % 4 == 0;
@@ -412,15 +416,6 @@ void layout_workspace(const kvb_paged_args* a, const Split& sp, char* base, floa
     *part_ml = reinterpret_cast<float2*>(base + slots * (size_t)a->head_dim * sizeof(float));
 }
 
-// Microseconds that a lone workgroup takes for one round of its four waves (128 tokens), which the
-// latency of its loads and its arithmetic set, not the card's bandwidth: from steps of 40 to 100
-// workgroups on MI355X at partitions of 1024 tokens and more.
-float round_us(int kind, int head_dim, bool fast) {
-    const bool d64 = head_dim == 64;
-    const float t = kind == KVB_KV_I8 ? (d64 ? 1.1f : 0.95f) : kind == KVB_KV_F16 ? (d64 ? 1.1f : 1.5f) : (d64 ? 1.9f : 3.4f);
-    return fast ? t : 1.25f * t;  // (any page size: per-lane addresses and scales)
-}
-
 // The partition where the caller leaves it to the library (part_tokens 0) and the library owns the
 // workspace: kvb_auto_part_tokens, or an even split of at most `part` tokens, a multiple of kEvenTokens
 // and larger than that (so that the workspace sized for the former holds it).
@@ -429,19 +424,40 @@ float round_us(int kind, int head_dim, bool fast) {
 // and its share of the merge then cost as much as its tokens, and short steps are cut into pieces of
 // two waves' work. The rule here takes the candidate with the least estimated time, from what a step is
 // made of (us):
-//   all:   every item's bytes at the card's rate and kItemUs, spread over the CUs
-//   waves: the same in whole items per CU, as many as the fullest CU has
-//   alone: the longest item by itself, or the CUs' resident workgroups in turn, at round_us
+//   waves: every item's bytes at the card's rate and kItemUs, in whole items per CU, as many as the
+//          fullest CU has; of a ragged batch, whose CUs start their next item as one ends, spread
+//          over the CUs with a share of the longest item at the end
+//   alone: the longest item by itself, or the CUs' resident workgroups in turn, at alone_us
 //   merge: none for one partition; past 16 partitions its longer form
-// The constants minimise the loss against the fastest candidate in a sweep of 62 shapes (batch 1-72,
-// 66-32768 tokens, equal and ragged, groups 1-64, all types, pages 8-64; up to 25 candidates each): 1.4%
-// on average, where kvb_auto_part_tokens loses 16%. E.g. (us, auto / this / best) fp16 1 x 4096:
-// 17.4 / 10.0 / 10.0; fp16 2 x 32768: 51.4 / 46.0 / 46.0; int8 72 ragged up to 16384: 252 / 212 / 208; its
-// worst: fp16 64 ragged up to 2048: 56.4 / 59.2 / 52.5; fp32 8 ragged up to 2048: 20.4 / 23.0 / 20.4.
+// The constants minimise the loss against the fastest candidate, and what is slower than under
+// kvb_auto_part_tokens, over 1007 shapes (batch 1-300, 64-32768 tokens, equal and ragged, groups 1-64, all
+// types, pages 1-256), repeated and after a flush: 1.8% off the fastest on average, where
+// kvb_auto_part_tokens is 14%; 49 shapes are slower than under it by more than 2%, the worst by 16% (fp32, 6 x
+// 1313 tokens, 16 KV heads: 29.2 us, 34.1). E.g. (us, auto / this) fp16 1 x 32768, one KV head, 115 / 17.3; fp32
+// 64 ragged up to 2048, 89 / 89; int8 24 ragged up to 6000, 16 KV heads, head_dim 64, page 24, 58 / 49.
+//
+// A candidate must also be one whose sums are no less exact than with 512 tokens, the most that
+// kvb_auto_part_tokens takes, and whose block ids fit in LDS on the any-page path (page 1, fp32, 16 x 32768
+// tokens: 4096-token partitions 199 us, 8192, whose ids do not, 864). fp16 and int8 waves add up a
+// partition's tiles one by one (2-norm against 64 bits, fp16 at head_dim 64 and 128, partitions of 512,
+// 1024, 1536, 2048 and 4096 tokens: 2.71, 2.71, 2.76, 2.93, 3.34e-7 and 2.89, 2.89, 2.98, 3.07, 3.47e-7; int8
+// 4.94, 4.95, 4.98, 5.08, 5.29e-7 and 5.03, 5.02, 5.05, 5.10, 5.33e-7); fp32's error does not grow (4.56e-7 at
+// 512, 4.50e-7 at 4096).
+constexpr int kEvenMost16 = 1024, kEvenMost32 = 4096;
+
+// Microseconds that a lone workgroup takes for 128 tokens, one round of its four waves, which the latency of
+// its loads and its arithmetic set, not the card's bandwidth.
+float round_us(int kind, int head_dim, bool fast) {
+    const bool d64 = head_dim == 64;
+    const float t = kind == KVB_KV_I8 ? (d64 ? 1.057f : 1.446f) : kind == KVB_KV_F16 ? (d64 ? 1.018f : 1.93f) : (d64 ? 2.49f : 3.091f);
+    return fast ? t : t * (kind == KVB_KV_I8 ? 0.877f : kind == KVB_KV_F16 ? 0.956f : 1.275f);
+}
+
 Split split_of(const kvb_paged_args* a) {
-    constexpr float kItemUs = 1.5f, kAloneUs = 4.0f, kWavesShare = 0.9f, kRate = 27.0e3f;  // kRate: bytes per us and CU
-    // candidates, in kEvenTokens: every one up to 8, then 4 (3 past 4096 tokens) to a factor of 2
-    constexpr int kSteps[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48, 64, 80, 96, 128};
+    constexpr float kItemUs = 1.427f, kAloneUs = 3.507f, kRate = 25.56e3f;  // kRate: bytes per us and CU
+    constexpr float kAuto = 0.98f;  // (kvb_auto_part_tokens unless another is estimated 2% faster)
+    // candidates, in kEvenTokens
+    constexpr int kSteps[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32};
     Split sp{resolve_part(a), max_parts_of(a), false};
     if (a->part_tokens != 0 || a->workspace || a->batch <= 0) return sp;
     const int32_t* lens = a->host_seq_lens;
@@ -454,21 +470,22 @@ Split split_of(const kvb_paged_args* a) {
         equal = equal && lens[b] == lens[0];
     }
     if (longest == 0 || (!equal && a->batch > kvbk::kRaggedMaxBatch)) return sp;
+    const bool f32 = a->kv_type == KVB_KV_F32, i8 = a->kv_type == KVB_KV_I8, fast = a->page_size % kvbk::kTile == 0;
     const int groups = a->num_heads / query_heads_per_group(a), seqs = equal ? 1 : a->batch;
     const float units = (float)groups * (equal ? (float)a->batch : 1.0f), cus = (float)g.cus;
-    const int esz = a->kv_type == KVB_KV_F32 ? 4 : a->kv_type == KVB_KV_F16 ? 2 : 1;
     const float tokens = (float)total * (float)groups;
-    const float token_us = 2.0f * a->head_dim * esz / kRate;
-    const float alone_us = round_us(a->kv_type, a->head_dim, a->page_size % kvbk::kTile == 0) / kvbk::kEvenTokens;
-    const float resident = a->kv_type == KVB_KV_I8 ? 3.0f : 2.0f;  // workgroups per CU
+    const float token_us = 2.0f * a->head_dim * (f32 ? 4 : i8 ? 1 : 2) / kRate;
+    const float alone_us = round_us(a->kv_type, a->head_dim, fast) / kvbk::kEvenTokens;
     // (partitions of 64 tokens leave two of the four waves idle: only fp32, whose tiles are twice fp16's,
     // is ever the faster for them)
-    const bool keep = a->kv_type == KVB_KV_F32 || sp.part >= kvbk::kEvenTokens;
+    const bool keep = f32 || sp.part >= kvbk::kEvenTokens;
     float best = 0.0f;
     int part = 0;
     for (int i = keep ? -1 : 0; i < (int)std::size(kSteps); ++i) {  // -1: kvb_auto_part_tokens
         const int cand = i < 0 ? sp.part : kSteps[i] * kvbk::kEvenTokens;
         if (i >= 0 && cand <= sp.part) continue;
+        const int blocks = cand / a->page_size + 2;
+        if (part != 0 && (cand > (f32 ? kEvenMost32 : kEvenMost16) || (!fast && blocks > kvbk::kTableStage))) break;
         // (an estimate: the counts in floating point, summed as integers so that the loop vectorises)
         const float inv = 1.0f / (float)cand;
         int n_all = 0, most_i = 0;
@@ -480,14 +497,23 @@ Split split_of(const kvb_paged_args* a) {
         }
         const float items = (float)n_all * units;
         const int grain = std::min(cand, kvbk::kEvenTokens);
-        const float most = std::min((float)((most_i + grain - 1) / grain * grain), (float)longest);
+        const float most = std::min(i < 0 ? (float)cand : (float)((most_i + grain - 1) / grain * grain), (float)longest);
         const float mean = tokens / items;
-        const float all = (tokens * token_us + items * kItemUs) / cus;
-        const float waves = items > cus ? std::ceil(items / cus) * (mean * token_us + kItemUs) : most * token_us + kItemUs;
-        const float alone = std::max(most * alone_us + kAloneUs, items / (cus * resident) * (mean * alone_us + kAloneUs));
+        // workgroups per CU (fewer where they stage many block ids)
+        const bool staged = !fast && a->kv_type != KVB_KV_F16 && blocks > kvbk::kTableStageSmall;
+        const float resident = i8 ? (staged ? 1.454f : 3.52f) : staged && a->head_dim == 128 ? 1.0f : 1.523f;
+        const float item_us = mean * token_us + kItemUs;
+        const float turns_us = items / (cus * resident) * (mean * alone_us + kAloneUs);
+        float waves = most * token_us + kItemUs, alone = std::max(most * alone_us + kAloneUs, turns_us);
+        if (items > cus && equal) {
+            waves = std::ceil(items / cus) * item_us;
+        } else if (items > cus) {
+            waves = 0.96f * items / cus * item_us + 0.211f * most * token_us;
+            alone = std::max(alone, 0.729f * turns_us + 1.5f * most * alone_us);
+        }
         const float parts = std::ceil((float)longest * inv);
-        const float merge = parts <= 1.0f ? 0.0f : parts <= 8.0f ? 1.5f : parts <= 16.0f ? 2.0f : 4.5f + 0.03f * (parts - 16.0f);
-        const float est = std::max(all * (1.0f - kWavesShare) + waves * kWavesShare, alone) + merge;
+        const float merge = parts <= 1.0f ? 0.0f : parts <= 8.0f ? 1.604f : parts <= 16.0f ? 1.915f : 3.218f + 0.1842f * (parts - 16.0f);
+        const float est = (std::max(waves, alone) + merge) * (i < 0 ? kAuto : 1.0f);
         if (part == 0 || est < best) {
             best = est;
             part = cand;
@@ -568,6 +594,11 @@ int kvb_paged_kernel_name(const kvb_paged_args* a, int loads_only, char* buf, si
     mk.step.describe = buf;
     mk.step.describe_cap = cap;
     return enqueue_paged(a, split_of(a), nullptr, nullptr, !loads_only, mk, loads_only != 0);
+}
+
+int kvb_paged_part_tokens(const kvb_paged_args* a) {
+    if (validate_paged(a) != KVB_OK || ensure_device() != KVB_OK) return -1;
+    return split_of(a).part;
 }
 
 int kvb_run_empty_grid(int workgroups, int threads, double* ms) {

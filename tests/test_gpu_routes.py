@@ -122,3 +122,30 @@ def test_wide_groups_on_few_workgroups(gpu, kv, group, dim, batch, heads):
     dev = kvb.DeviceCase(w, c)
     assert build_of(kvb, dev, 256)["heads"] == str(heads)
     dev.free()
+
+
+# page, sequences, their length: fewer and fuller workgroups than at 512 tokens would suit the batch
+LONG = [(1, 16, 32768), (1, 32, 16384), (1, 64, 8192), (3, 16, 32768), (24, 64, 8192), (64, 64, 8192)]
+
+
+@pytest.mark.parametrize("kv,most", [("f32", 4096), ("f16", 1024), ("i8", 1024)])
+@pytest.mark.parametrize("page,batch,n", LONG)
+@pytest.mark.parametrize("ragged", [False, True])
+def test_library_partitions_stay_exact_and_staged(gpu, kv, most, page, batch, n, ragged):
+    """Left to the library, no partition is so long that its error grows or that its block ids no longer fit
+    in LDS (by the lengths alone: nothing is launched, so the pool need not hold them)."""
+    kvb = gpu
+    w = kvb.Workload(kvb.Shape(batch, 16, 2, 128), kv, [24] * batch, seed=1)
+    c = kvb.PagedCache(w, page, 1)
+    dev = kvb.DeviceCase(w, c)
+    a = dev.args(0)
+    lens = np.array([n - 5 * i * ragged for i in range(batch)], np.int32)
+    a.max_len, a.max_blocks, a.host_seq_lens = n, -(-n // page), lens.ctypes.data
+    part = kvb.hip.kvb_paged_part_tokens(ctypes.byref(a))
+    assert 0 < part <= most
+    buf = ctypes.create_string_buffer(512)
+    kvb.check(kvb.hip.kvb_paged_kernel_name(ctypes.byref(a), 0, buf, 512), "paged_kernel_name")
+    values = dict(zip(FIELDS, buf.value.decode().split("<")[1].split(">")[0].split(", ")))
+    if page % 16:
+        assert values["stage"] != "0" and part // page + 2 <= 4096
+    dev.free()
