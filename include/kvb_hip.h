@@ -182,7 +182,10 @@ int kvb_run_paged_steps(const kvb_paged_args* a, int steps, double* ms);
  * their shapes while it exists. The captured steps are the same kernels, in the same order, as
  * kvb_run_paged_steps: the same bits. They allocate nothing and contain no memset node. The grid
  * and the work order are fixed at capture from host_seq_lens. Equal lengths at capture (the plain
- * grid): each replay serves the device seq_lens as they are then, clamped to the captured max_len.
+ * grid): each replay serves the device seq_lens as they are then, clamped to the captured max_len. At
+ * part_tokens 0 the partition is chosen at capture too: a shorter sequence is cut into up to as many
+ * partitions as the captured length, a longer one into more, and the sums may run in another order than
+ * in an eager step, which chooses for the lengths it is given.
  * Lengths not all equal (the longest-first order): every replay needs device seq_lens equal to the
  * captured host_seq_lens; lengths that make a different number of work items turn the replay into a
  * no-op that leaves out as it was and reports no error. Same refusals as kvb_run_paged, plus

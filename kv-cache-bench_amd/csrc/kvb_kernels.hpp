@@ -82,11 +82,19 @@ __device__ __forceinline__ int fast_div(int n, FastDiv f) {
 // partial. Even: as many partitions as part_tokens tokens each would need, all of one size but the
 // last (a multiple of kEvenTokens, so that every wave of a workgroup gets as many tiles), so that no
 // short remainder is left: the library's choice where the caller leaves the partition to it (runtime.hip).
+// That choice is made for the host's lengths. Where they are equal (the plain grid), a captured step may be
+// replayed at shorter ones: a sequence that part_tokens would cut into fewer than `parts`, its partitions at
+// the host's length, is cut by `nominal` (kvb_auto_part_tokens) into at most that many, so that the grid is not
+// left idle (one KV head, fp16, captured at 32768 tokens in partitions of 512 and replayed at 1000: 8
+// partitions, not 2).
 constexpr int kEvenTokens = 128;
 struct SplitParams {
     int part_tokens;
     int even;
     FastDiv part_div;           // division by part_tokens
+    int parts = 0;              // 0: part_tokens alone
+    int nominal = 0;
+    FastDiv nominal_div;
 };
 // Tokens per partition of a sequence of len tokens, 1 <= len; ceil(len / that) <= ceil(len / part_tokens).
 __host__ __device__ __forceinline__ int even_part(int len, int n) {
@@ -94,7 +102,10 @@ __host__ __device__ __forceinline__ int even_part(int len, int n) {
                   : ((len + n - 1) / n + kEvenTokens - 1) / kEvenTokens * kEvenTokens;
 }
 __device__ __forceinline__ int seq_part(const SplitParams& s, int len) {
-    return s.even ? even_part(len, fast_div(len + s.part_tokens - 1, s.part_div)) : s.part_tokens;
+    if (!s.even) return s.part_tokens;
+    int n = fast_div(len + s.part_tokens - 1, s.part_div);
+    if (n < s.parts) n = min(s.parts, fast_div(len + s.nominal - 1, s.nominal_div));
+    return even_part(len, n);
 }
 
 struct DecodeParams {

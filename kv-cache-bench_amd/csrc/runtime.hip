@@ -165,6 +165,7 @@ struct Split {
     int part;       // tokens per partition, or (even) at most that many
     int max_parts;  // partitions of max_len tokens: the workspace's stride, the plain grid's z
     bool even;      // SplitParams::even
+    int parts = 0;  // SplitParams::parts: partitions of each sequence, where all are as long
 };
 Split split_of(const kvb_paged_args* a);
 
@@ -340,7 +341,9 @@ int enqueue_paged(const kvb_paged_args* a, const Split& sp, float* part_out, flo
     p.max_blocks = a->max_blocks;
     p.max_parts = sp.max_parts;
     p.part_tokens = part;
-    p.split = {part, sp.even ? 1 : 0, kvbk::make_fast_div((uint32_t)part)};
+    const int nominal = resolve_part(a);
+    p.split = {part, sp.even ? 1 : 0, kvbk::make_fast_div((uint32_t)part),
+               sp.parts, nominal, kvbk::make_fast_div((uint32_t)nominal)};
     p.len_cap = len_cap_of(a, sp);
     p.qscale = (1.0f / std::sqrt((float)a->head_dim)) * 1.4426950408889634f;
     p.batch = a->batch;
@@ -521,7 +524,8 @@ Split split_of(const kvb_paged_args* a) {
         if (cand >= longest) break;
     }
     if (part <= sp.part) return sp;
-    return Split{part, std::max(1, (int)(((long long)a->max_len + part - 1) / part)), true};
+    return Split{part, std::max(1, (int)(((long long)a->max_len + part - 1) / part)), true,
+                 equal ? (longest + part - 1) / part : 0};
 }
 
 int workspace_for(const kvb_paged_args* a, const Split& sp, float** part_out, float2** part_ml) {

@@ -7,6 +7,7 @@ import ctypes
 import numpy as np
 import pytest
 
+import parity_battery as pb
 from conftest import progress
 
 pytestmark = pytest.mark.gpu
@@ -62,6 +63,45 @@ def test_graph_replays_match_eager(gpu):
     finally:
         for dev, _, _ in devs:
             dev.free()
+
+
+@pytest.mark.parametrize("kv", ["f32", "f16", "i8"])
+@pytest.mark.parametrize("heads,n,page", [((8, 1, 64), 4096, 16), ((4, 2, 128), 3000, 24)])
+def test_replays_at_other_lengths_keep_their_partitions(gpu, oracle, kv, heads, n, page):
+    """A step whose partition is the library's, captured at one length: shorter replays are cut into about as
+    many partitions as that length, not into pieces of its size, so that they are no longer than an eager step's.
+    The bits are those of an explicit partition of the same size."""
+    kvb = gpu
+    w = kvb.Workload(kvb.Shape(2, *heads), kv, [n] * 2, seed=n, q_amp=2.0, varied=(kv == "i8"))
+    c = kvb.PagedCache(w, page, 13, pool_factor=1.5)
+    dev = kvb.DeviceCase(w, c)
+    graph = None
+    try:
+        dev.out.fill(0xFF)
+        dev.run(0)
+        fresh = dev.output()
+        parts, nominal = -(-n // dev.part_tokens(0)), kvb.auto_part_tokens(2, heads[1], n)
+        graph = dev.capture_graph(0, 1)
+        for short in (1000, 129, n - 1, 1, n):
+            lens = np.array([short, n], np.int32)
+            dev.lens.upload(lens)
+            dev.out.fill(0xFF)
+            graph.launch()
+            got = dev.output()
+            assert np.array_equal(got[1], fresh[1])
+            w.lens = lens
+            pb.check_output(kvb, oracle, w, c, got)
+            count = -(-short // dev.part_tokens(0))
+            if count < parts:
+                count = min(parts, -(-short // nominal))
+            even = -(-(-(-short // count)) // 128) * 128
+            dev.out.fill(0xFF)
+            dev.run(even)
+            assert np.array_equal(got[0], dev.output()[0]), f"{short} tokens in partitions of {even}"
+    finally:
+        if graph is not None:
+            graph.free()
+        dev.free()
 
 
 def test_graph_refusals(gpu):
