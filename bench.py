@@ -202,7 +202,7 @@ def main():
     ap.add_argument("--warmup", type=int, default=3)
     ap.add_argument("--config", default="c4", choices=sorted(WORKLOAD_TEXT))
     ap.add_argument("--part", type=int, default=None,
-                    help="partition tokens (default: the config's, else the MI355X policy; 0 = auto_part_tokens)")
+                    help="partition tokens (default: the config's, else the MI355X policy; 0 = the library's choice)")
     ap.add_argument("--pair", choices=["auto", "off", "always"], default="auto",
                     help="two partitions per decode workgroup (kvb_set_pair_mode); the same bits either way")
     ap.add_argument("--no-cpu", action="store_true")
@@ -245,8 +245,8 @@ def main():
         wi = kvb.Workload(w.shape, "i8", list(w.lens), seed=32768, q_amp=1.0, dist="normal", threads=cpu_threads())
         ci = kvb.PagedCache(wi, 128, 32768 * 131 + 128, pool_factor=1.25, poison=False)
         devi = kvb.DeviceCase(wi, ci)
-    nparts = dev.max_parts(part)
-    part_res = kvb.auto_part_tokens(w.shape.batch, w.shape.num_kv_heads, w.max_len) if part == 0 else part
+    part_res = dev.part_tokens(part)
+    nparts = -(-w.max_len // part_res)
     log(f"{args.config} ready in {time.perf_counter() - t_setup:.1f}s: {int(w.lens.sum())} tokens, "
         f"pool {c.num_blocks} blocks, partition {part_res} ({nparts} per sequence)")
 

@@ -121,7 +121,7 @@ int kvb_auto_part_tokens(int batch, int num_kv_heads, int max_len);
  * resolved as kvb_run_paged does (src/metal_attn.mm:160-161). Returns -1 on bad arguments. */
 int kvb_paged_max_parts(const kvb_paged_args* a);
 /* Not in the reference: tokens per partition of kvb_run_paged's step with these arguments; at part_tokens 0
- * without a workspace, the most that one of the library's even cut holds. Same refusals as kvb_run_paged
+ * without a workspace, those of the sequence that the library cuts into the largest. Same refusals as kvb_run_paged
  * (-1, kvb_last_error); launches nothing. */
 int kvb_paged_part_tokens(const kvb_paged_args* a);
 /* Bytes of the workspace a call with these arguments uses (0 on bad arguments). */

@@ -29,6 +29,7 @@
 #include <functional>
 #include <map>
 #include <span>
+#include <stdexcept>
 #include <string>
 #include <thread>
 #include <vector>
@@ -361,7 +362,13 @@ std::vector<float> gpu_fp64(const Workload& w) {
     return std::vector<float>(p, p + w.out_floats());
 }
 
-int resolved_part(const Workload& w, int part) { return part ? part : auto_part_tokens(w.shape, w.max_len); }
+// The partition a step runs with, for its row: the library's own where --parts has 0.
+int part_of_step(const PagedArgs& a) {
+    const kvb_paged_args c = c_args(a);
+    const int part = kvb_paged_part_tokens(&c);
+    if (part < 0) throw std::runtime_error(kvb_last_error());
+    return part;
+}
 
 // ---- modes -----------------------------------------------------------------------------------------
 
@@ -555,8 +562,8 @@ int mode_sweep(const Options& o, const GpuTimer& timer, const CpuReference& cpu_
             for (int page : o.pages) {
                 const PagedCache cache(w, page, uint64_t(L) * 131 + page, false, o.pool, false);
                 for (int part : o.parts) {
-                    const int p = resolved_part(w, part);
                     const PagedArgs args = cache.args(w, part, out_paged);
+                    const int p = part_of_step(args);
                     const Sample s = timer([&] { return run_paged(args); });
                     const double diff = have_naive ? max_abs_diff(out_paged.as<float>(), out_naive.as<float>(), n) : NAN;
                     if (o.flush) flush_gpu_caches();
@@ -571,7 +578,7 @@ int mode_sweep(const Options& o, const GpuTimer& timer, const CpuReference& cpu_
                         PagedArgs one = args;
                         one.share_kv = false;
                         const Sample sp = timer([&] { return run_paged(one); });
-                        timed("gpu_paged_per_head", w, page, p, o.reps, sp)
+                        timed("gpu_paged_per_head", w, page, part_of_step(one), o.reps, sp)
                             .general("max_diff_vs_naive",
                                      have_naive ? max_abs_diff(out_paged.as<float>(), out_naive.as<float>(), n) : NAN)
                             .count("kv_bytes", (long long)cache.bytes())

@@ -246,12 +246,15 @@ struct StepMarks {
     kvbk::Marks step, decode, reduce;
 };
 
-// Partitions of a sequence of len tokens.
-long long parts_of(int len, const Split& sp) {
+// Tokens per partition of a sequence of the host's len tokens, and its partitions.
+long long part_of(int len, const Split& sp) {
     if (len <= 0) return 0;
-    long long part = sp.part;
-    if (sp.even) part = kvbk::even_part(len, (int)(((long long)len + sp.part - 1) / sp.part));
-    return (len + part - 1) / part;
+    if (!sp.even) return sp.part;
+    return kvbk::even_part(len, (int)(((long long)len + sp.part - 1) / sp.part));
+}
+long long parts_of(int len, const Split& sp) {
+    const long long part = part_of(len, sp);
+    return part ? (len + part - 1) / part : 0;
 }
 
 // Workgroups of a step that hold tokens.
@@ -602,7 +605,11 @@ int kvb_paged_kernel_name(const kvb_paged_args* a, int loads_only, char* buf, si
 
 int kvb_paged_part_tokens(const kvb_paged_args* a) {
     if (validate_paged(a) != KVB_OK || ensure_device() != KVB_OK) return -1;
-    return split_of(a).part;
+    const Split sp = split_of(a);
+    if (!sp.even) return sp.part;
+    long long most = 1;
+    for (int b = 0; b < a->batch; ++b) most = std::max(most, part_of(a->host_seq_lens[b], sp));
+    return (int)most;
 }
 
 int kvb_run_empty_grid(int workgroups, int threads, double* ms) {

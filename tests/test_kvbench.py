@@ -129,6 +129,26 @@ def test_kvbench_sweep_loads_and_cpu_rows(gpu):
 
 
 @pytest.mark.gpu
+def test_kvbench_rows_name_the_partition_that_ran(gpu):
+    """A row for --parts=0 carries the size the library chose, not the reference's rule."""
+    kvb = gpu
+    out = subprocess.run([KVBENCH, "--batch=1", "--lens=700,4096", "--pages=16", "--parts=0,512", "--reps=1",
+                          "--warmup=0", "--types=f16,i8"], capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0, out.stderr
+    rows = [r for r in csv_rows(out.stdout)[1] if r["impl"] == "gpu_paged"]
+    assert len(rows) == 8
+    for i, r in enumerate(rows):
+        n = int(r["seq_len"])
+        if i % 2:
+            assert r["part"] == "512"
+            continue
+        w = kvb.Workload(kvb.Shape(1, 32, 8, 128), r["dtype"], [n], seed=1)
+        dev = kvb.DeviceCase(w, kvb.PagedCache(w, 16, 1))
+        assert int(r["part"]) == dev.part_tokens(0) != kvb.auto_part_tokens(1, 8, n)
+        dev.free()
+
+
+@pytest.mark.gpu
 def test_kvbench_chain(gpu):
     """--chain=N (bench/bench.cpp:155-185): per type, a contiguous and a paged16 row; max_err against
     fp64 on the stored values (f32, f16: within the kernel tolerance 2e-5) or on the unquantised data
