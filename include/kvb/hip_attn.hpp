@@ -59,9 +59,10 @@ inline size_t elem_size(KvType t) { return t == KvType::f32 ? 4 : t == KvType::f
 // have 4 wave64s, one per SIMD, for every storage type.
 constexpr int kSimdGroups = 4;
 
-// Split-K partition size used when PagedArgs::part_tokens is 0 (src/metal_attn.hpp:43-51): the
+// The reference's split-K partition size for PagedArgs::part_tokens 0 (src/metal_attn.hpp:43-51): the
 // largest power of two in [64, 512] that still yields at least 512 (sequence, KV head,
-// partition) triples.
+// partition) triples. Here 0 leaves the size to the library, which takes this one or an even cut into
+// larger partitions, never into more (kvb_paged_part_tokens).
 inline int auto_part_tokens(const Shape& s, int max_len) {
     int part = 512;
     while (part > 64 && size_t(s.batch) * s.num_kv_heads * ((max_len + part - 1) / part) < 512) part /= 2;
@@ -110,7 +111,7 @@ struct PagedArgs {
     int page_size = 16;
     int max_blocks = 0;      // PagedLayout::max_blocks
     int max_len = 0;         // longest sequence, sizes the split-K workspace; 0: all empty, out is 0
-    int part_tokens = 0;     // split-K partition size, 0 = auto_part_tokens()
+    int part_tokens = 0;     // split-K partition size, 0 = the library's choice
     const Buffer* q;         // float [B][H][D]
     const Buffer* k;         // type  [blocks][Hkv][page][D]
     const Buffer* v;

@@ -118,7 +118,8 @@ typedef struct kvb_paged_args {
  * the largest power of two in [64, 512] with batch * Hkv * ceil(max_len / part) >= 512. */
 int kvb_auto_part_tokens(int batch, int num_kv_heads, int max_len);
 /* Partitions per (sequence, head) in the workspace: max(1, ceil(max_len / part)) with part
- * resolved as kvb_run_paged does (src/metal_attn.mm:160-161). Returns -1 on bad arguments. */
+ * part_tokens, or kvb_auto_part_tokens() at 0 (src/metal_attn.mm:160-161): at 0 without a workspace a step
+ * has at most as many. Returns -1 on bad arguments. */
 int kvb_paged_max_parts(const kvb_paged_args* a);
 /* Not in the reference: tokens per partition of kvb_run_paged's step with these arguments; at part_tokens 0
  * without a workspace, those of the sequence that the library cuts into the largest. Same refusals as kvb_run_paged
@@ -135,7 +136,10 @@ size_t kvb_paged_workspace_bytes(const kvb_paged_args* a);
  * and a workgroup of 32 heads splits them over two sets of waves that walk the same tiles (f16:
  * each tile loaded once and shared through LDS). A step of at most 16 partitions per sequence whose
  * workgroups of 16 or 32 heads would leave half the CUs idle runs workgroups of 8 or 16 heads
- * instead. Returns -1 on bad arguments
+ * instead (8 for 16 heads of an int8 cache at head_dim 64 only where seven CUs of eight would be idle).
+ * Workgroups of 8 and of 16 heads sum a partition in different orders, so the output of a group of 16
+ * or 32 may differ in its last bits (2e-7 of its size) with how many sequences share its step, and
+ * with the lengths of the others. Returns -1 on bad arguments
  * (num_kv_heads <= 0, num_heads not a positive multiple of it, kv_type not a kvb_kv_type). */
 int kvb_heads_per_workgroup(int num_heads, int num_kv_heads, int kv_type, int share_kv);
 
@@ -221,7 +225,8 @@ int kvb_paged_kernel_name(const kvb_paged_args* a, int loads_only, char* buf, si
  * instead of one. KVB_PAIR_AUTO (the default): when the plain (sequence, partition) grid would put
  * two or more workgroups on every CU; KVB_PAIR_OFF: never; KVB_PAIR_ALWAYS: whenever it is allowed.
  * It is allowed for f16 and i8 caches with page_size and the partition multiples of 16, the
- * partition a multiple of 128, at least two partitions, and equal lengths (or one sequence). Every
+ * partition a multiple of 128, at least two partitions, and equal lengths (or one sequence), not for
+ * the even cut that part_tokens 0 may choose. Every
  * setting gives the same bits: each partition is computed by the same waves, in the same order.
  * Returns the previous setting, or -1 for an unknown one (nothing changed). Applies to every later
  * decode step of the process. */
