@@ -3,9 +3,9 @@ reference's scripts/env.sh, which saves machine, toolchain, commit and load besi
 
 `python3 build_info.py OUT` (run by the package Makefile) writes OUT, a JSON record of the build: the
 git commit and whether tracked files differed from it, the sha256 of the sources the libraries are
-built from, the time and the hipcc version. The GPU box receives the tree without .git, so a result
+built from, the time and the hipcc version. A tree may be run without its .git, so a result
 measured there names its build through this file; `sources_sha256` recomputed at run time shows
-whether the sources on the box are the ones built.
+whether the sources beside it are the ones built.
 
 `env_record(kvb)` is the environment object of a bench line: that source identity, the HIP runtime
 and driver versions and the device (kvb_device_info), the ROCm release, the CPU and the load average
@@ -46,7 +46,7 @@ def sources_sha256() -> str:
 
 
 def git_state():
-    """(commit, dirty) from git, or (None, None) where there is no repository (the GPU box)."""
+    """(commit, dirty) from git, or (None, None) where there is no repository."""
     try:
         commit = subprocess.run(["git", "-C", ROOT, "rev-parse", "HEAD"], capture_output=True, text=True,
                                 timeout=10).stdout.strip()

@@ -50,7 +50,7 @@ def main(out):
     print("Workload: batch 4, 8 KV heads, head_dim 128, context 32768, page 128, partition 4096, cold (1 GiB read "
           "flush per step); q, K, V ~ U(-1, 1) from kvbench's seeds, K/V stored as fp16 (RNE) or int8 per-(page, KV "
           "head) scales; shuffled block table.\n")
-    print("## Commands (from the repository root on the GPU box)\n")
+    print("## Commands (from the repository root on an MI355X machine)\n")
     print("```\nbash kv-cache-bench_amd/bench/profile_groups.sh gpurun_out/prof_groups\n```\n")
     print("For each storage type t and group G (query heads H = 8 G), from /tmp with TMPDIR=/tmp (R = the repository "
           "root, A = `--batch=4 --heads=H --kv-heads=8 --dim=128 --lens=32768 --pages=128 --parts=4096 --types=t "

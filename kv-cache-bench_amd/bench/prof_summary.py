@@ -99,7 +99,7 @@ def main(cfg, out):
           f"{line['data']}.\n")
     print(f"Kernel: `{kname}` (grid {timed[0][1]['Grid_Size_X']} threads, {timed[0][1]['VGPR_Count']} arch VGPR + "
           f"{timed[0][1]['Accum_VGPR_Count']} AGPR, LDS {timed[0][1]['LDS_Block_Size']} B).\n")
-    print("## Commands (from the repository root on the GPU box)\n")
+    print("## Commands (from the repository root on an MI355X machine)\n")
     print("```")
     root = os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
     print(f"bash kv-cache-bench_amd/bench/profile.sh {cfg} {os.path.relpath(out, root)}")

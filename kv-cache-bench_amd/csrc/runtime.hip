@@ -281,8 +281,9 @@ int ragged_items(const kvb_paged_args* a, const Split& sp) {
 
 // Query heads per workgroup of this step: kvb_heads_per_workgroup, but 8 (or 16 of 32) where the
 // workgroups of the wider kind would leave at least half the CUs idle. A KV head's workgroups then run on
-// CUs of their own (one XCD, so that the later reads of a page come from its L2), instead of as one
-// whose waves spend two or four heads' arithmetic per tile in turn; every head's sums are the same, to
+// CUs of their own (on one XCD, so that the later reads of a page come from its L2, where the units of a step
+// come in eights; else each reads the pages for itself: 8 ragged up to 8192 tokens, group 32, fetch 54 MiB for
+// 26), instead of as one whose waves spend two or four heads' arithmetic per tile in turn; every head's sums are the same, to
 // fp32 rounding (16 of 32: to the bit). us, one 32- or 16-head workgroup / two or more: fp16 1 x 8192
 // tokens, one KV head, 512-token partitions, 32 heads 19.8 / 11.5, 16 heads 13.2 / 11.2; fp16 8 ragged up
 // to 8192, 2 KV heads, 32 heads 23.0 / 17.5; int8 2 x 2048, 8 KV heads, 16 heads 12.7 / 10.9; 1 x 65536

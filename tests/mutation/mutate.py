@@ -13,7 +13,7 @@ Groups:
           of this build's split-K kernel (kvbo_split_decode in oracle/kvb_oracle.c, which uses the
           kernel's number formats). They are checked by tests/test_split_model.py, which is the GPU
           parity battery (tests/parity_battery.py) run on that model. No deliberately broken kernel
-          runs on a GPU (the GPU boxes forbid it); group hip runs the kernel's own source mutated,
+          runs on a GPU; group hip runs the kernel's own source mutated,
           on the CPU emulation.
   hip     mistakes planted in the shipped kernels' own source (paged_decode_impl.hpp and its
           headers, paged_reduce, the cache writer): the arithmetic of the MFMA kernel (the q and p
