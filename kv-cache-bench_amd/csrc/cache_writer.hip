@@ -21,7 +21,6 @@ namespace kvbk {
 namespace {
 
 constexpr int kWriterThreads = 256;
-constexpr int kScatterWords = 2;
 constexpr long long kStreamBytes = 128ll << 20;  // read and written
 
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
@@ -33,13 +32,14 @@ __device__ __forceinline__ u32x4_t load_word(const u32x4_t* p) {
     else return *p;
 }
 
-// A workgroup copies kWriterThreads * kScatterWords 16-byte words of consecutive tokens (8 KB: 32
-// fp16 rows at head_dim 128) of one (KV head, sequence), whatever the page size: the loads do not wait
-// for the block ids, which each lane looks up for its own rows while they are in flight. (1, 2 and 4
-// words per thread: 2 is the fastest or within 4% of it from 0.2 MB to 1 GB.)
+// A workgroup copies kWriterThreads * U 16-byte words of consecutive tokens (U 2, 8 KB: 32 fp16 rows at
+// head_dim 128) of one (KV head, sequence), whatever the page size: the loads do not wait for the block
+// ids, which each lane looks up for its own rows while they are in flight. (1, 2 and 4 words per thread: 2
+// is the fastest or within 4% of it from 0.2 MB to 1 GB; of the calls that stream, 4 by 1-2%.)
+constexpr int scatter_words(bool stream) { return stream ? 4 : 2; }
 template <bool STREAM>
 __global__ __launch_bounds__(kWriterThreads) void scatter_kernel(CacheWriteParams p) {
-    constexpr int U = kScatterWords;
+    constexpr int U = scatter_words(STREAM);
     const int kvh = blockIdx.x, b = blockIdx.y;
     const int len = live_len(p.seq_lens, b, p.len_cap);
     const int shift = p.row_shift, tokens = (kWriterThreads * U) >> shift;
@@ -209,7 +209,7 @@ hipError_t launch_write_paged(const CacheWriteParams& p, int batch, int max_bloc
         else launch_quantize<false>(p, batch, max_blocks_used, s, m);
         return hipGetLastError();
     }
-    const int tokens = (kWriterThreads * kScatterWords) >> p.row_shift;
+    const int tokens = (kWriterThreads * scatter_words(stream)) >> p.row_shift;
     const long long runs = (p.max_len + (long long)tokens - 1) / tokens;
     const dim3 grid(p.num_kv_heads, batch, (unsigned)(runs < 65535 ? runs : 65535)), block(kWriterThreads);
     if (stream) launch_marked(scatter_kernel<true>, grid, block, s, m, p);
