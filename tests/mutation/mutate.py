@@ -247,6 +247,23 @@ MUTANTS = [
       "ml[j] = p.part_ml[i];\n            v[j] = p.part_out[base * D + d];", "kv-cache-bench_amd/csrc/kernels_misc.hip"),
     X("cache writer: int8 quantiser truncates",
       "__builtin_rintf(x / scale)", "truncf(x / scale)", "kv-cache-bench_amd/csrc/cache_writer.hip"),
+    X("even cut: a partition more than the host counts",
+      "return even_part(len, n);", "return even_part(len, n + 1);", "kv-cache-bench_amd/csrc/kvb_kernels.hpp"),
+    X("even cut: a shorter replay keeps the captured partition",
+      "if (n < s.parts) n = min(", "if (n < s.parts) (void)min(", "kv-cache-bench_amd/csrc/kvb_kernels.hpp"),
+    X("even cut: fp16 and int8 partitions of up to 4096 tokens",
+      "kEvenMost16 = 1024", "kEvenMost16 = 4096", RUNTIME),
+    X("narrow workgroups of a wide group on twice the CUs",
+      "share * workgroups(a, sp, 2 * few) <= g.cus", "share * workgroups(a, sp, 2 * few) <= 2 * g.cus", RUNTIME),
+    X("int8, any page: the staged scales of the range's first page for every token",
+      "return s_sc[fast_div(t < t1 ? t : t0, p.page_div) - tb0];", "return s_sc[0 * t];"),
+    X("fp32 walk: the refilled K rows are the present tile's",
+      "load_rows(r[0], tn, std::true_type{}, std::false_type{});",
+      "load_rows(r[0], tn - TS * kTok, std::true_type{}, std::false_type{});"),
+    X("naive P.V: a chunk's weights relative to its own max",
+      "__expf(sc[t] - mx) * inv", "__expf(sc[t] - st[chunk].x) * inv", "kv-cache-bench_amd/csrc/kernels_misc.hip"),
+    X("naive sum drops the last chunk",
+      "o += c0 + j < nch ? x[j]", "o += c0 + j < nch - 1 ? x[j]", "kv-cache-bench_amd/csrc/kernels_misc.hip"),
     # ---- the checker ----
     O("fp64 reference has no case for an empty sequence (scripts/mutation.sh:36)",
       "len ? (float)(acc[d] / sum) : 0.0f", "(float)(acc[d] / sum)"),
