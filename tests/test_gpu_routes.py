@@ -149,3 +149,20 @@ def test_library_partitions_stay_exact_and_staged(gpu, kv, most, page, batch, n,
     if page % 16:
         assert values["stage"] != "0"
     dev.free()
+
+
+# page, partition, the build's table: a block either side of what each holds
+@pytest.mark.parametrize("kv", ["f32", "f16", "i8"])
+@pytest.mark.parametrize("page,part,table", [(1, 512, 512), (1, 513, 4096), (1, 4096, 4096), (1, 4097, 0),
+                                             (3, 1536, 512), (3, 1537, 4096), (3, 1529, 512)])
+def test_block_ids_at_the_edges_of_their_tables(gpu, oracle, kv, page, part, table):
+    kvb = gpu
+    lens = [part + 130, part, 1]
+    w = kvb.Workload(kvb.Shape(len(lens), 4, 1, 64), kv, lens, seed=part, varied=(kv == "i8"))
+    c = kvb.PagedCache(w, page, part, pool_factor=1.1, poison=True)
+    dev = kvb.DeviceCase(w, c)
+    assert build_of(kvb, dev, part)["stage"] == str(4096 if table and kv == "f16" else table)  # (fp16: one table)
+    dev.out.fill(0xFF)
+    dev.run(part)
+    pb.check_output(kvb, oracle, w, c, dev.output())
+    dev.free()
